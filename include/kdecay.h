@@ -122,6 +122,27 @@ int kdecay_scan_fwd(const void* V, int v_dtype, const int64_t* v_strides,
 size_t kdecay_scan_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t D,
                                    int v_dtype);
 
+/*
+ * kdecay_scan_fwd for every head dim and alignment: the same arguments,
+ * results, workspace rules and error handling (its workspace is
+ * kdecay_scan_rows_workspace_bytes() bytes and may be the same buffer), but D
+ * is any number of channels of at least one 16-byte vector (8 bf16/fp16, 4
+ * fp32, 2 fp64), and V, out and the other strides need the element type's
+ * alignment only (d-stride 1).  Streams are whole rows of up to 256 bytes; it
+ * is for the arrays kdecay_scan_fwd refuses, which is the faster one for
+ * those it takes.
+ */
+int kdecay_scan_fwd_rows(const void* V, int v_dtype, const int64_t* v_strides,
+                         void* out, int out_dtype, const int64_t* out_strides,
+                         const float* lam, const float* init_state,
+                         float* final_state, int64_t B, int64_t H, int64_t N,
+                         int64_t D, int64_t t_offset, void* workspace,
+                         size_t workspace_bytes, void* stream);
+
+/* Bytes of workspace kdecay_scan_fwd_rows needs for this shape (0: none). */
+size_t kdecay_scan_rows_workspace_bytes(int64_t B, int64_t H, int64_t N,
+                                        int64_t D, int v_dtype);
+
 /* Size of the fixed device array kdecay_scan_fwd_noalloc uses as workspace. */
 #define KDECAY_NOALLOC_WORKSPACE_BYTES ((size_t)8 << 20)
 

@@ -1,4 +1,4 @@
-"""Build recipe of ``libkdecay.so``: one hipcc invocation for gfx950.
+"""Build recipe of ``libkdecay.so``: one hipcc compilation per source for gfx950, then a link.
 
 Run ``python -m kilat_amd._build`` (or ``__graft_entry__.build()``).  The
 library is written in-tree next to this file, where ``kilat_amd._lib`` loads it.
@@ -9,10 +9,11 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
-SOURCE = os.path.join(HERE, "csrc", "kdecay.hip")
+SOURCES = [os.path.join(HERE, "csrc", name) for name in ("kdecay.hip", "kdecay_rows.hip")]
 INCLUDE = os.path.join(ROOT, "include")
 LIBRARY = os.path.join(HERE, "libkdecay.so")
 
@@ -25,7 +26,6 @@ HIPCC_FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-mcode-object-version=5",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
@@ -39,20 +39,31 @@ def hipcc() -> str:
 
 
 def build_library(verbose: bool = False) -> str:
-    """Compile csrc/kdecay.hip into libkdecay.so; returns the library path."""
-    tmp = LIBRARY + ".tmp"
-    cmd = [hipcc(), *HIPCC_FLAGS, "-I", INCLUDE, SOURCE, "-o", tmp]
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    # hipcc's host pass does not know the packed-fp32 target feature and says
-    # so; that line is expected and not shown.
-    lines = [l for l in proc.stdout.splitlines() if "packed-fp32-ops" not in l and l.strip()]
-    if proc.returncode != 0:
-        raise RuntimeError("hipcc failed:\n" + "\n".join(lines))
-    if verbose and lines:
-        print("\n".join(lines), flush=True)
-    os.replace(tmp, LIBRARY)
+    """Compile the csrc sources into libkdecay.so; returns the library path."""
+    with tempfile.TemporaryDirectory(prefix="kdecay_build_") as work:
+        jobs = []  # the sources compile side by side
+        for src in SOURCES:
+            obj = os.path.join(work, os.path.basename(src) + ".o")
+            cmd = [hipcc(), *HIPCC_FLAGS, "-I", INCLUDE, "-c", src, "-o", obj]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            jobs.append((obj, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+        done = [(obj, proc.communicate()[0], proc.returncode) for obj, proc in jobs]
+        tmp = LIBRARY + ".tmp"
+        if all(rc == 0 for _, _, rc in done):
+            cmd = [hipcc(), "--offload-arch=gfx950", "-shared", *[obj for obj, _, _ in done], "-o", tmp]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+            done.append((tmp, proc.stdout, proc.returncode))
+        # hipcc's host pass does not know the packed-fp32 target feature and says
+        # so; that line is expected and not shown.
+        lines = [l for _, out, _ in done for l in out.splitlines() if "packed-fp32-ops" not in l and l.strip()]
+        if any(rc != 0 for _, _, rc in done):
+            raise RuntimeError("hipcc failed:\n" + "\n".join(lines))
+        if verbose and lines:
+            print("\n".join(lines), flush=True)
+        os.replace(tmp, LIBRARY)
     return LIBRARY
 
 

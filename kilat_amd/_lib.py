@@ -32,6 +32,8 @@ KDECAY_NOALLOC_WORKSPACE_BYTES = 8 << 20  # include/kdecay.h
 EXPORTS = (
     "kdecay_scan_fwd",
     "kdecay_scan_workspace_bytes",
+    "kdecay_scan_fwd_rows",
+    "kdecay_scan_rows_workspace_bytes",
     "kdecay_scan_fwd_noalloc",
     "kdecay_scan_fwd_train",
     "kdecay_scan_saved_states_floats",
@@ -75,6 +77,10 @@ def load() -> ctypes.CDLL:
     ]
     lib.kdecay_scan_workspace_bytes.restype = ctypes.c_size_t
     lib.kdecay_scan_workspace_bytes.argtypes = [_c_i64, _c_i64, _c_i64, _c_i64, ctypes.c_int]
+    lib.kdecay_scan_fwd_rows.restype = ctypes.c_int
+    lib.kdecay_scan_fwd_rows.argtypes = lib.kdecay_scan_fwd.argtypes
+    lib.kdecay_scan_rows_workspace_bytes.restype = ctypes.c_size_t
+    lib.kdecay_scan_rows_workspace_bytes.argtypes = lib.kdecay_scan_workspace_bytes.argtypes
     lib.kdecay_scan_fwd_noalloc.restype = ctypes.c_int
     lib.kdecay_scan_fwd_noalloc.argtypes = [
         _c_ptr, ctypes.c_int, _c_i64p,      # V, v_dtype, v_strides

@@ -38,9 +38,10 @@ _GROUP = {torch.float32: 32, torch.bfloat16: 64, torch.float16: 64, torch.float6
 
 def chunked_head_dim(D: int, dtype: torch.dtype) -> bool:
     """Head dims the chunked kernels take as they are: 16, 32, or a multiple of
-    one 128-byte channel group (64 bf16/fp16, 32 fp32 or 16 fp64 channels).  Other head
-    dims are zero-padded to the next such size on the way in (channels are
-    independent, so the padding changes no value) and sliced on the way out."""
+    one 128-byte channel group (64 bf16/fp16, 32 fp32 or 16 fp64 channels).
+    Others take the row kernel (_rows) or, where that does not apply, are
+    zero-padded to the next such size on the way in (channels are independent,
+    so the padding changes no value) and sliced on the way out."""
     return D == 16 or D == 32 or (D > 0 and D % _GROUP[dtype] == 0)
 
 
@@ -51,6 +52,21 @@ def _padded_head_dim(D: int, dtype: torch.dtype) -> int:
         return 32
     full = _GROUP[dtype]
     return -(-D // full) * full
+
+
+def _row_vectors_ok(D: int, dtype: torch.dtype) -> bool:
+    """Head dims kdecay_scan_fwd_rows splits into 16-byte vectors (row_split in
+    kdecay_rows.hip): whole rows of up to 16 vectors, wider ones in the fewest
+    equal streams; not less than one vector, and not a last stream of one
+    vector that overlaps the stream before it."""
+    vw = _GROUP[dtype] // 8
+    if D < vw:
+        return False
+    nv = -(-D // vw)
+    ng = -(-nv // 16)
+    left = nv - (ng - 1) * -(-nv // ng)
+    return left >= 1 and (ng == 1 or left >= 2 or D % vw == 0)
+
 
 # One zero-initialised workspace per (device, stream); the kernels keep it
 # consistent from launch to launch, so it is never cleared again.
@@ -128,13 +144,14 @@ def _on_device(device: torch.device):
 _ws_bytes_cache: dict = {}
 
 
-def _fwd_workspace_bytes(lib, B: int, H: int, N: int, D: int, v_code: int) -> int:
-    key = (B, H, N, D, v_code)
+def _fwd_workspace_bytes(lib, B: int, H: int, N: int, D: int, v_code: int, rows: bool = False) -> int:
+    key = (B, H, N, D, v_code, rows)
     n = _ws_bytes_cache.get(key)
     if n is None:
         if len(_ws_bytes_cache) > 1024:
             _ws_bytes_cache.clear()
-        n = _ws_bytes_cache[key] = lib.kdecay_scan_workspace_bytes(B, H, N, D, v_code)
+        size = lib.kdecay_scan_rows_workspace_bytes if rows else lib.kdecay_scan_workspace_bytes
+        n = _ws_bytes_cache[key] = size(B, H, N, D, v_code)
     return n
 
 
@@ -176,7 +193,10 @@ def reserve_workspace(
         dev = torch.device("cuda", torch.cuda.current_device())
     code = _dtype_code(torch.empty((), dtype=dtype), "dtype")
     lib = _lib.load()
-    nbytes = lib.kdecay_scan_workspace_bytes(B, H, N, D, code)
+    if chunked_head_dim(D, dtype):
+        nbytes = lib.kdecay_scan_workspace_bytes(B, H, N, D, code)
+    else:
+        nbytes = lib.kdecay_scan_rows_workspace_bytes(B, H, N, D, code)
     if backward:
         # float64 is trained through the fp32 kernels (_scan_with_grad)
         tcode = _lib.KDECAY_F32 if code == _lib.KDECAY_F64 else code
@@ -332,8 +352,9 @@ def global_decay_scan(
     Returns y ([B,H,N,D], dtype out_dtype or V.dtype, laid out like V), and
     with return_final_state also s_{N-1} ([B,H,D] fp32).
     algorithm: "chunked" (default) or "sequential" (the cross-check kernel).
-    Head dims the chunked kernels do not take (chunked_head_dim) are
-    zero-padded to the next one they do.  When lam, V or initial_state
+    Head dims and layouts the chunked kernels do not take (chunked_head_dim) run
+    on the row kernel, rows of less than 16 bytes zero-padded to the next head
+    dim the chunked kernels take.  When lam, V or initial_state
     requires grad, the result carries a backward for every head dim, layout,
     algorithm and out= (the gradients always come from the chunked backward
     kernel).  The backward kernel takes the upstream gradient in V's dtype:
@@ -380,6 +401,10 @@ def global_decay_scan(
                 final.data_ptr() if final is not None else None, B, H, N, D, int(t_offset), stream,
             )
             _lib.check(rc, "kdecay_scan_fwd_sequential")
+        elif chunked_head_dim(D, V.dtype) and _vector_layout_ok(V) and _vector_layout_ok(out):
+            _chunked(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev)
+        elif _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev):
+            pass
         elif chunked_head_dim(D, V.dtype):
             _chunked(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev)
         else:  # zero channels up to a head dim the chunked kernels take
@@ -420,6 +445,36 @@ def _chunked(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream
     _lib.check(rc, "kdecay_scan_fwd")
     if outk is not out:
         out.copy_(outk)
+
+
+def _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev) -> bool:
+    """kdecay_scan_fwd_rows on V into out, for the head dims and alignments
+    kdecay_scan_fwd refuses.  False, with nothing launched, where it does not
+    apply: rows of less than one 16-byte vector, and a stream being captured
+    whose workspace holds less than this route needs (the callers' fallback
+    may need less, or allocates what it needs inside the capture)."""
+    B, H, N, D = V.shape
+    if not _row_vectors_ok(D, V.dtype):
+        return False
+    nbytes = _fwd_workspace_bytes(lib, B, H, N, D, v_code, rows=True)
+    ws = _workspaces.get((dev.index, stream))
+    if (nbytes if ws is None else nbytes - ws.numel()) > 0 and torch.cuda.is_current_stream_capturing():
+        return False
+    Vk = V if V.stride(3) == 1 else V.contiguous()
+    outk = out if out.stride(3) == 1 else torch.empty(V.shape, dtype=out.dtype, device=dev)
+    ws = _workspace(dev, stream, nbytes)
+    rc = lib.kdecay_scan_fwd_rows(
+        Vk.data_ptr(), v_code, _lib.strides4(Vk.stride()),
+        outk.data_ptr(), o_code, _lib.strides4(outk.stride()),
+        lam32.data_ptr(), init32.data_ptr() if init32 is not None else None,
+        final.data_ptr() if final is not None else None, B, H, N, D, int(t_offset),
+        ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0,
+        stream,
+    )
+    _lib.check(rc, "kdecay_scan_fwd_rows")
+    if outk is not out:
+        out.copy_(outk)
+    return True
 
 
 def _scan_with_grad(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, algorithm):

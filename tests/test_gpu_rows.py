@@ -1,0 +1,159 @@
+"""The row kernel (kdecay_scan_fwd_rows): head dims and alignments the
+channel-group kernels refuse, against the oracle and the sequential kernel."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+import kilat_amd
+from kilat_amd import _lib
+from kilat_amd.triton_ops import _row_vectors_ok, chunked_head_dim
+from oracle import decay_oracle as O
+from tests.decay_cases import lam_uniform, rel_err
+
+DTYPES = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16, "f64": torch.float64}
+CODES = {"f32": _lib.KDECAY_F32, "bf16": _lib.KDECAY_BF16, "f16": _lib.KDECAY_F16, "f64": _lib.KDECAY_F64}
+# The fp32 values differ in their last bits (1e-5 of the stream's largest), and
+# where that moves one across a rounding boundary the 2-byte outputs differ by
+# one ulp: 2^-8 to 2^-7 of the value for bf16 (8 significant bits), 2^-11 to
+# 2^-10 for fp16 (11).
+TOL = {torch.float32: 1e-5, torch.bfloat16: 1e-5 + 2.0 ** -7, torch.float16: 1e-5 + 2.0 ** -10, torch.float64: 1e-5}
+
+
+@pytest.mark.parametrize("dname", ["f32", "bf16", "f16", "f64"])
+def test_row_split_agrees_with_the_library(kdecay_lib, dname):
+    """The shim's rule for which head dims the row kernel takes is the
+    library's: it sizes a workspace for exactly those (several chunks here)."""
+    for D in range(1, 700):
+        ok = kdecay_lib.kdecay_scan_rows_workspace_bytes(2, 3, 100000, D, CODES[dname]) > 0
+        assert ok == _row_vectors_ok(D, DTYPES[dname]), D
+
+
+def test_rows_rejects_bad_arguments(kdecay_lib):
+    fake = 0x100000
+    ok = (3 * 4096 * 50, 4096 * 50, 50, 1)
+
+    def call(V=fake, D=50, vstr=ok, ws=fake, wsb=1 << 30, code=_lib.KDECAY_BF16, ocode=_lib.KDECAY_BF16):
+        return kdecay_lib.kdecay_scan_fwd_rows(V, code, _lib.strides4(vstr), fake, ocode, _lib.strides4(ok), fake, None,
+                                               None, 2, 3, 4096, D, 0, ws, wsb, None)
+
+    assert call(V=None) == _lib.KDECAY_EINVAL
+    assert call(V=fake + 1) == _lib.KDECAY_ELAYOUT  # not on an element boundary
+    assert call(vstr=(3 * 4096 * 100, 4096 * 100, 100, 2)) == _lib.KDECAY_ELAYOUT
+    assert call(D=7) == _lib.KDECAY_ESHAPE  # less than one 16-byte vector
+    assert call(code=9) == _lib.KDECAY_EDTYPE
+    assert call(ocode=_lib.KDECAY_F16) == _lib.KDECAY_EDTYPE
+    assert call(ws=None, wsb=0) == _lib.KDECAY_EWORKSPACE
+    assert call(wsb=64) == _lib.KDECAY_EWORKSPACE
+    assert call(ws=fake + 8) == _lib.KDECAY_EWORKSPACE
+
+
+def _check(lam, V, dev, out_dtype=None, init=None, offset=0, out=None):
+    lam_d, V_d = lam.to(dev), V.to(dev)
+    if V_d.stride() != V.stride():
+        V_d = torch.empty_strided(V.shape, V.stride(), dtype=V.dtype, device=dev).copy_(V)
+    kw = dict(initial_state=None if init is None else init.to(dev), t_offset=offset, return_final_state=True,
+              out_dtype=out_dtype)
+    y, fin = kilat_amd.global_decay_scan(lam_d, V_d, **kw)
+    yseq, fseq = kilat_amd.global_decay_scan(lam_d, V_d, algorithm="sequential", **kw)
+    assert y.shape == V.shape and y.stride() == yseq.stride()
+    tol = TOL[y.dtype]
+    assert rel_err(y, yseq) <= tol and rel_err(fin, fseq) <= 1e-5
+    if V.numel() <= 1 << 20:
+        ref, sref = O.scan(lam, V.float() if V.dtype == torch.float64 else V, init, offset,
+                           out_dtype=torch.float32 if y.dtype == torch.float64 else y.dtype)
+        assert rel_err(y, ref) <= tol and rel_err(fin, sref) <= 1e-5
+    return y
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname,D", [
+    ("bf16", 8), ("bf16", 9), ("bf16", 15), ("f16", 24), ("bf16", 33), ("f16", 40), ("bf16", 48), ("bf16", 50),
+    ("f16", 80), ("bf16", 96), ("bf16", 100), ("f16", 127),  # one stream per head, 1 to 16 lanes
+    ("bf16", 129), ("bf16", 136), ("f16", 160), ("bf16", 264), ("bf16", 301),  # two and three streams, surplus lanes
+    ("f32", 4), ("f32", 5), ("f32", 20), ("f32", 50), ("f32", 63), ("f32", 68), ("f32", 100),
+    ("f64", 2), ("f64", 3), ("f64", 20), ("f64", 33), ("f64", 50),
+])
+def test_rows_head_dims(hip_device, kdecay_lib, dname, D):
+    """Every number of lanes per row; sequences of one row, around the end of a
+    chunk of 8 rows per lane, and of several chunks; both layouts."""
+    dtype = DTYPES[dname]
+    assert _row_vectors_ok(D, dtype) and not chunked_head_dim(D, dtype)
+    g = torch.Generator().manual_seed(900 + D)
+    lam = lam_uniform(3, 0.5, 0.9999, g)
+    vw = 16 // torch.empty((), dtype=dtype).element_size()
+    nv = -(-D // vw)
+    lpr = -(-nv // -(-nv // 16))
+    L = 4 * (64 // lpr) * 8
+    for N in (1, L - 1, L, L + 1, 5 * L + 3):
+        for tokens in (False, True):
+            V = torch.randn(2, N, 3, D, generator=g).to(dtype).transpose(1, 2)
+            V = V if tokens else V.contiguous()
+            init = torch.randn(2, 3, D, generator=g) if tokens else None
+            _check(lam, V, hip_device, init=init, offset=7 if tokens else 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname,out,B,H,N,D", [
+    ("bf16", None, 24, 16, 1500, 96),    # 16 rows per lane, several rounds
+    ("f16", None, 8, 16, 2047, 80),      # one round
+    ("bf16", "f32", 16, 9, 2000, 72),    # fp32 outputs, two stores per row
+    ("f32", None, 16, 16, 1024, 40),
+    ("bf16", None, 40, 10, 700, 50),     # 400 streams: counted through sub-counts
+    ("f16", None, 1, 2, 30000, 40),      # a long chain: the wide window
+    ("bf16", None, 130, 16, 60, 48),     # many short sequences
+])
+def test_rows_grids(hip_device, kdecay_lib, dname, out, B, H, N, D):
+    g = torch.Generator().manual_seed(950 + D)
+    lam = lam_uniform(H, 0.5, 0.9999, g)
+    V = torch.randn(B, H, N, D, generator=g).to(DTYPES[dname])
+    y1 = _check(lam, V, hip_device, out_dtype=DTYPES[out] if out else None)
+    y2 = _check(lam, V, hip_device, out_dtype=DTYPES[out] if out else None)
+    assert torch.equal(y1, y2)  # the same bits on every run
+
+
+@pytest.mark.gpu
+def test_rows_misaligned_views_and_out(hip_device, kdecay_lib):
+    """D=64 (a head dim of the channel-group kernels) on bases and row strides
+    off the 16-byte grid, and with out given: misaligned, with a channel
+    stride, and V itself (written in place)."""
+    g = torch.Generator().manual_seed(77)
+    lam = lam_uniform(4, 0.8, 0.999, g).to(hip_device)
+    big = torch.randn(2, 4, 900, 67, generator=g).to(torch.bfloat16).to(hip_device)
+    for V in (big[..., 1:65], big[..., 3:53], big[:, :, 1::2, 2:66]):
+        ref = kilat_amd.global_decay_scan(lam, V, algorithm="sequential")
+        y = kilat_amd.triton_global_decay(lam, V)
+        assert rel_err(y, ref) <= TOL[torch.bfloat16]
+        room = torch.zeros(*V.shape[:3], V.shape[3] + 3, dtype=V.dtype, device=hip_device)
+        out = room[..., 1:-2]
+        assert kilat_amd.global_decay_scan(lam, V, out=out) is out and torch.equal(out, y)
+        assert not room[..., 0].any() and not room[..., -2:].any()  # nothing written beside the rows
+        wide = torch.zeros(*V.shape[:3], 2 * V.shape[3], dtype=V.dtype, device=hip_device)
+        kilat_amd.global_decay_scan(lam, V, out=wide[..., ::2])
+        assert torch.equal(wide[..., ::2], y) and not wide[..., 1::2].any()
+        W = V.clone()
+        kilat_amd.global_decay_scan(lam, W, out=W)
+        assert rel_err(W, ref) <= TOL[torch.bfloat16]
+
+
+@pytest.mark.gpu
+def test_rows_under_capture(hip_device, kdecay_lib):
+    """Captured after reserve_workspace and replayed between eager calls of
+    other shapes on the same workspace; on a stream whose workspace is too
+    small for the row kernel the capture still takes what it took before it."""
+    g = torch.Generator().manual_seed(78)
+    lam = lam_uniform(3, 0.8, 0.999, g).to(hip_device)
+    V = torch.randn(2, 3, 3000, 80, generator=g).to(torch.bfloat16).to(hip_device)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert kilat_amd.triton_ops.reserve_workspace(2, 3, 3000, 80, torch.bfloat16, backward=False) > 0
+        ref = kilat_amd.triton_global_decay(lam, V)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            y = kilat_amd.triton_global_decay(lam, V)
+        for _ in range(3):
+            y.zero_()
+            graph.replay()
+            kilat_amd.triton_global_decay(lam, V[:, :, :1000, :64])
+            side.synchronize()
+            assert torch.equal(y, ref)

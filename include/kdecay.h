@@ -284,6 +284,38 @@ size_t kdecay_scan_bwd_workspace_bytes(int64_t B, int64_t H, int64_t N,
                                        int64_t D, int v_dtype);
 
 /*
+ * The training forward and the backward of kdecay_scan_fwd_rows: as
+ * kdecay_scan_fwd_train and kdecay_scan_bwd, with that entry point's head dims,
+ * strides (any, also negative row strides) and alignment.  The states buffer is
+ * kdecay_scan_rows_saved_states_floats() floats, B*H*D per backward chunk plus
+ * 2*H*N row terms, and goes to kdecay_scan_rows_bwd only.
+ */
+int kdecay_scan_fwd_rows_train(const void* V, int v_dtype,
+                               const int64_t* v_strides, void* out,
+                               int out_dtype, const int64_t* out_strides,
+                               const float* lam, const float* init_state,
+                               float* final_state, float* states,
+                               size_t states_floats, int64_t B, int64_t H,
+                               int64_t N, int64_t D, int64_t t_offset,
+                               void* workspace, size_t workspace_bytes,
+                               void* stream);
+
+size_t kdecay_scan_rows_saved_states_floats(int64_t B, int64_t H, int64_t N,
+                                            int64_t D, int v_dtype);
+
+int kdecay_scan_rows_bwd(const void* V, int v_dtype, const int64_t* v_strides,
+                         const void* gy, const int64_t* gy_strides, void* dV,
+                         const int64_t* dv_strides, const float* lam,
+                         const float* init_state, const float* states,
+                         const float* g_final, float* dlam, float* d_init,
+                         int64_t B, int64_t H, int64_t N, int64_t D,
+                         int64_t t_offset, void* workspace,
+                         size_t workspace_bytes, void* stream);
+
+size_t kdecay_scan_rows_bwd_workspace_bytes(int64_t B, int64_t H, int64_t N,
+                                            int64_t D, int v_dtype);
+
+/*
  * Incremental (decode) step for a whole batch, one launch.
  * Replaces the inline update
  *   new_state = lam.view(1,H,1) * past_state + V_current

@@ -34,6 +34,10 @@ EXPORTS = (
     "kdecay_scan_workspace_bytes",
     "kdecay_scan_fwd_rows",
     "kdecay_scan_rows_workspace_bytes",
+    "kdecay_scan_fwd_rows_train",
+    "kdecay_scan_rows_saved_states_floats",
+    "kdecay_scan_rows_bwd",
+    "kdecay_scan_rows_bwd_workspace_bytes",
     "kdecay_scan_fwd_noalloc",
     "kdecay_scan_fwd_train",
     "kdecay_scan_saved_states_floats",
@@ -117,6 +121,12 @@ def load() -> ctypes.CDLL:
     ]
     lib.kdecay_scan_bwd_workspace_bytes.restype = ctypes.c_size_t
     lib.kdecay_scan_bwd_workspace_bytes.argtypes = [_c_i64, _c_i64, _c_i64, _c_i64, ctypes.c_int]
+    for name in ("kdecay_scan_fwd_train", "kdecay_scan_saved_states_floats", "kdecay_scan_bwd",
+                 "kdecay_scan_bwd_workspace_bytes"):
+        fn = getattr(lib, name)
+        rows = getattr(lib, {"kdecay_scan_fwd_train": "kdecay_scan_fwd_rows_train"}.get(
+            name, name.replace("scan_", "scan_rows_")))
+        rows.restype, rows.argtypes = fn.restype, fn.argtypes
     lib.kdecay_scan_fwd_sequential.restype = ctypes.c_int
     lib.kdecay_scan_fwd_sequential.argtypes = [
         _c_ptr, ctypes.c_int, _c_i64p,

@@ -933,70 +933,9 @@ struct ChunkBwd {
     // stream's first chunk before its dV pass (as the forward counts its
     // last chunks) takes the count off the launch's tail: 0.5-2% faster.
     if (rc == a.nchunk - 1 && b == a.B - 1 && grp == a.ng - 1)
-      reduce_head(a, h, epoch, poisoned);
+      reduce_head<SL>(a, h, epoch, poisoned);
     else if (!a.per_stream && item + kXcds >= (int)gridDim.x && tid == 0 && !poisoned)
       count_done(a.hdr, (unsigned)a.ndone, epoch);
-  }
-
-  // dlam[h] = the sum of head h's chunk partials in double, in a fixed order
-  // whatever the order in which they arrive (deterministic): wavefront 0
-  // alone, each lane summing a strided subset (all its reads issued at
-  // once), then a fixed butterfly across the lanes.
-  __device__ static void reduce_head(const BwdArgs& a, int h, unsigned epoch, bool poisoned) {
-    if (threadIdx.x >= 64) return;
-    const int lane = threadIdx.x;
-    const unsigned tag = tag_of(epoch, 0u);
-    const int n = (int)a.B * a.ng * a.nchunk;
-    constexpr int K = 8;
-    double acc = 0.0;
-    for (int i0 = 0; i0 < n; i0 += 64 * K) {
-      const u64* p[K];
-      u64 w[K];
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const int idx = i0 + lane + 64 * k < n ? i0 + lane + 64 * k : n - 1;
-        const int bg = (int)a.f_nchunk.div((uint32_t)idx), rc = idx - bg * a.nchunk;
-        const int b = (int)a.f_ng.div((uint32_t)bg), grp = bg - b * a.ng;
-        p[k] = a.partial + (int64_t)rc * a.nstream + ((int64_t)b * a.H + h) * a.ng + grp;
-        w[k] = peek(p[k]);
-      }
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        if (i0 + lane + 64 * k >= n) continue;
-        for (int spin = 0; (unsigned)(w[k] >> 32) != tag; ++spin) {
-          if (spin >= a.spin_limit) {  // give up: flag it, and the head's dlam becomes NaN
-            __hip_atomic_store(a.hdr + HDR_ERROR, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            w[k] = ((u64)tag << 32) | 0x7fc00000u;
-            break;
-          }
-          __builtin_amdgcn_s_sleep(1);
-          w[k] = peek(p[k]);
-        }
-        acc += (double)__uint_as_float((unsigned)w[k]);
-      }
-    }
-    acc = wave_sum_f64(acc);
-    if (lane == 0) {
-      // Only the batch-slice kernels carry this (compiled into every kernel,
-      // it cost one more VGPR, and five waves per SIMD, in the 4-row
-      // narrow-group kernels and 1.2% at the B=8 N=4096 H=12 backward).
-      if constexpr (SL) {
-        if (a.slice + 1 < a.nslice) {
-          a.dlam_slices[(int64_t)a.slice * a.H + h] = acc;  // the last slice adds it
-        } else {
-          double t = acc;
-          if (a.slice > 0) {  // the earlier slices' sums in slice order, then this one's
-            t = a.dlam_slices[h];
-            for (int sl = 1; sl < a.slice; ++sl) t += a.dlam_slices[(int64_t)sl * a.H + h];
-            t += acc;
-          }
-          a.dlam[h] = (float)t;
-        }
-      } else {
-        a.dlam[h] = (float)acc;
-      }
-      if (!a.per_stream && !poisoned) count_done(a.hdr, (unsigned)a.ndone, epoch);
-    }
   }
 };
 
@@ -1539,13 +1478,6 @@ constexpr int kRB = 16;
 constexpr int kRBSmall = 4;
 constexpr int kNWB = 4;
 constexpr int64_t kBwdSmallGrid = 256;
-// Streams up to which every stream's first chunk counts toward the epoch's
-// advance (ChunkBwd::run).  Measured (bf16, same-box A/B, per stream / per
-// head and XCD, us): D=64 B=8 N=1024 H=6 (48 streams) 11.13 / 11.48; B=8
-// N=4096 H=12 (96) 28.77 / 29.17; B=12 N=2048 H=16 (192) 29.31 / 29.61;
-// B=16 N=2048 H=16 (256) 40.68 / 40.86; B=16 N=1024 H=16 (256) 23.96 /
-// 23.21; B=24 N=1024 H=16 (384) 37.23 / 29.21.
-constexpr int64_t kBwdPerStreamCount = 192;
 constexpr int64_t kBwdShortChainGrid = 384;
 
 // 4 rows per lane when the 16-row grid has at most kBwdSmallGrid chunks, so
@@ -1732,6 +1664,33 @@ int empty_final_state(const float* init, float* fin, int64_t n, hipStream_t s) {
   if (!fin || n == 0) return 0;
   hipLaunchKernelGGL(copy_state, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, init, fin, n);
   return hip_check("copy_state launch");
+}
+
+// Backward of an empty sequence: the gradients are the final-state gradient
+// passed through.
+int empty_backward(const float* g_final, float* d_init, float* dlam, int64_t B, int64_t H, int64_t D, hipStream_t s) {
+  hipLaunchKernelGGL(copy_state, dim3((unsigned)((B * H * D + 255) / 256)), dim3(256), 0, s, g_final, d_init,
+                     d_init ? B * H * D : 0);
+  const int e = hip_check("copy_state launch");
+  if (e) return e;
+  hipLaunchKernelGGL(zero_floats, dim3((unsigned)((H + 255) / 256)), dim3(256), 0, s, dlam, H);
+  return hip_check("zero_floats launch");
+}
+
+// Workgroups of a backward launch that count toward the epoch's advance: the H
+// that sum a head's partials (the last row of items, chunk 0, is unrotated:
+// item (nchunk-1)*nstream + stream with b = B-1 and the last channel group) and
+// the last of each XCD, each counted once.
+int bwd_done_count(int64_t B, int64_t H, int64_t ng, int64_t nchunk) {
+  const int64_t nstream = B * H * ng, grid = nchunk * nstream;
+  int n = (int)H;
+  for (int64_t item = grid > kXcds ? grid - kXcds : 0; item < grid; ++item) {
+    const int64_t rc = item / nstream, stream = item - rc * nstream;
+    const int64_t bh = stream / ng, grp = stream - bh * ng;
+    const bool sums = rc == nchunk - 1 && bh / H == B - 1 && grp == ng - 1;
+    if (!sums) ++n;
+  }
+  return n;
 }
 
 }  // namespace kd
@@ -2002,14 +1961,7 @@ int kdecay_scan_bwd(const void* V, int v_dtype, const int64_t* v_strides, const 
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (B * H * D == 0) return 0;
   if (!lam || !dlam) return fail(KDECAY_EINVAL, "null pointer argument");
-  if (N == 0) {  // no rows: the gradients are the final-state gradient passed through
-    hipLaunchKernelGGL(copy_state, dim3((unsigned)((B * H * D + 255) / 256)), dim3(256), 0, s, g_final,
-                       d_init, d_init ? B * H * D : 0);
-    int e = hip_check("copy_state launch");
-    if (e) return e;
-    hipLaunchKernelGGL(zero_floats, dim3((unsigned)((H + 255) / 256)), dim3(256), 0, s, dlam, H);
-    return hip_check("zero_floats launch");
-  }
+  if (N == 0) return empty_backward(g_final, d_init, dlam, B, H, D, s);
   if (!V || !gy || !dV || !v_strides || !gy_strides || !dv_strides) return fail(KDECAY_EINVAL, "null pointer argument");
   if (!head_dim_ok(v_dtype, D))
     return fail(KDECAY_ESHAPE, "head dim D=%lld is not 16, 32 or a multiple of %d", (long long)D,
@@ -2086,18 +2038,8 @@ int kdecay_scan_bwd(const void* V, int v_dtype, const int64_t* v_strides, const 
     a.f_nchunk = make_fastdiv((uint32_t)nchunk);
     a.hdr = static_cast<unsigned*>(workspace);
     a.spin_limit = spin_limit();
-    // Workgroups that count toward the epoch's advance: the H that sum a
-    // head's partials (the last row of items, chunk 0, is unrotated: item
-    // (nchunk-1)*nstream + stream with b = B-1 and the last channel group) and
-    // the last of each XCD, each counted once.
     a.per_stream = nstream_s <= kBwdPerStreamCount;
-    a.ndone = (int)H;
-    for (int64_t item = grid_s > kXcds ? grid_s - kXcds : 0; item < grid_s; ++item) {
-      const int64_t rc = item / nstream_s, stream = item - rc * nstream_s;
-      const int64_t bh = stream / a.ng, grp = stream - bh * a.ng;
-      const bool sums = rc == nchunk - 1 && bh / H == Bs - 1 && grp == a.ng - 1;
-      if (!sums) ++a.ndone;
-    }
+    a.ndone = bwd_done_count(Bs, H, a.ng, nchunk);
     a.flags = nchunk > 1 ? reinterpret_cast<u64*>(static_cast<char*>(workspace) + kHeaderBytes) : nullptr;
     a.partial = reinterpret_cast<u64*>(static_cast<char*>(workspace) + kHeaderBytes + flag_bytes);
     a.slice = (int)i;

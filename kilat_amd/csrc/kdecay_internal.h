@@ -679,6 +679,69 @@ struct BwdArgs {
 // each XCD dispatches its share in index order.
 constexpr int kXcds = 8;
 
+// dlam[h] = the sum of head h's chunk partials in double, in a fixed order
+// whatever the order in which they arrive (deterministic): wavefront 0
+// alone, each lane summing a strided subset (all its reads issued at
+// once), then a fixed butterfly across the lanes.
+// SL: a launch over a batch slice (BwdArgs::nslice).
+template <bool SL>
+__device__ __forceinline__ void reduce_head(const BwdArgs& a, int h, unsigned epoch, bool poisoned) {
+  if (threadIdx.x >= 64) return;
+  const int lane = threadIdx.x;
+  const unsigned tag = tag_of(epoch, 0u);
+  const int n = (int)a.B * a.ng * a.nchunk;
+  constexpr int K = 8;
+  double acc = 0.0;
+  for (int i0 = 0; i0 < n; i0 += 64 * K) {
+    const u64* p[K];
+    u64 w[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int idx = i0 + lane + 64 * k < n ? i0 + lane + 64 * k : n - 1;
+      const int bg = (int)a.f_nchunk.div((uint32_t)idx), rc = idx - bg * a.nchunk;
+      const int b = (int)a.f_ng.div((uint32_t)bg), grp = bg - b * a.ng;
+      p[k] = a.partial + (int64_t)rc * a.nstream + ((int64_t)b * a.H + h) * a.ng + grp;
+      w[k] = peek(p[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (i0 + lane + 64 * k >= n) continue;
+      for (int spin = 0; (unsigned)(w[k] >> 32) != tag; ++spin) {
+        if (spin >= a.spin_limit) {  // give up: flag it, and the head's dlam becomes NaN
+          __hip_atomic_store(a.hdr + HDR_ERROR, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          w[k] = ((u64)tag << 32) | 0x7fc00000u;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+        w[k] = peek(p[k]);
+      }
+      acc += (double)__uint_as_float((unsigned)w[k]);
+    }
+  }
+  acc = wave_sum_f64(acc);
+  if (lane == 0) {
+    // Only the batch-slice kernels carry this (compiled into every kernel,
+    // it cost one more VGPR, and five waves per SIMD, in the 4-row
+    // narrow-group kernels and 1.2% at the B=8 N=4096 H=12 backward).
+    if constexpr (SL) {
+      if (a.slice + 1 < a.nslice) {
+        a.dlam_slices[(int64_t)a.slice * a.H + h] = acc;  // the last slice adds it
+      } else {
+        double t = acc;
+        if (a.slice > 0) {  // the earlier slices' sums in slice order, then this one's
+          t = a.dlam_slices[h];
+          for (int sl = 1; sl < a.slice; ++sl) t += a.dlam_slices[(int64_t)sl * a.H + h];
+          t += acc;
+        }
+        a.dlam[h] = (float)t;
+      }
+    } else {
+      a.dlam[h] = (float)acc;
+    }
+    if (!a.per_stream && !poisoned) count_done(a.hdr, (unsigned)a.ndone, epoch);
+  }
+}
+
 // --------------------------------------------------------------------------
 // Host helpers (kdecay.hip)
 // --------------------------------------------------------------------------
@@ -692,5 +755,15 @@ int cu_count();
 int check_scan_args(const void* V, int v_dtype, const int64_t* v_strides, const void* out, int out_dtype,
                     const int64_t* out_strides, const float* lam, int64_t B, int64_t H, int64_t N, int64_t D);
 int empty_final_state(const float* init, float* fin, int64_t n, hipStream_t s);
+int empty_backward(const float* g_final, float* d_init, float* dlam, int64_t B, int64_t H, int64_t D, hipStream_t s);
+int bwd_done_count(int64_t B, int64_t H, int64_t ng, int64_t nchunk);
+
+// Streams up to which every stream's first chunk counts toward the epoch's
+// advance (ChunkBwd::run).  Measured (bf16, same-box A/B, per stream / per
+// head and XCD, us): D=64 B=8 N=1024 H=6 (48 streams) 11.13 / 11.48; B=8
+// N=4096 H=12 (96) 28.77 / 29.17; B=12 N=2048 H=16 (192) 29.31 / 29.61;
+// B=16 N=2048 H=16 (256) 40.68 / 40.86; B=16 N=1024 H=16 (256) 23.96 /
+// 23.21; B=24 N=1024 H=16 (384) 37.23 / 29.21.
+constexpr int64_t kBwdPerStreamCount = 192;
 
 }  // namespace kd

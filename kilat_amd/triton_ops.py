@@ -200,8 +200,8 @@ def reserve_workspace(
     if backward:
         # float64 is trained through the fp32 kernels (_scan_with_grad)
         tcode = _lib.KDECAY_F32 if code == _lib.KDECAY_F64 else code
-        nbytes = max(nbytes, lib.kdecay_scan_workspace_bytes(B, H, N, D, tcode),
-                     lib.kdecay_scan_bwd_workspace_bytes(B, H, N, D, tcode))
+        tdtype = torch.float32 if code == _lib.KDECAY_F64 else dtype
+        nbytes = max(nbytes, _train_sizes(lib, B, H, N, D, tcode, not chunked_head_dim(D, tdtype))[1])
     with _on_device(dev):
         ws = _workspace(dev, _stream_ptr(dev), nbytes)
     return 0 if ws is None else ws.numel()
@@ -237,6 +237,34 @@ def _lam32(lam: torch.Tensor, H: int, device: torch.device) -> torch.Tensor:
     return lam.detach().reshape(H).to(device=device, dtype=torch.float32).contiguous()
 
 
+def _train_layout_ok(t: torch.Tensor) -> bool:
+    return _vector_layout_ok(t) and _bwd_rows_fit(t)
+
+
+def _row_layout_ok(t: torch.Tensor) -> bool:
+    """The row kernels' layout rule: d-stride 1."""
+    return t.stride(3) == 1
+
+
+def _train_sizes(lib, B: int, H: int, N: int, D: int, v_code: int, rows: bool) -> Tuple[int, int]:
+    """Floats of the saved states, and bytes of workspace that the training
+    forward and its backward need."""
+    if rows:
+        return (lib.kdecay_scan_rows_saved_states_floats(B, H, N, D, v_code),
+                max(lib.kdecay_scan_rows_workspace_bytes(B, H, N, D, v_code),
+                    lib.kdecay_scan_rows_bwd_workspace_bytes(B, H, N, D, v_code)))
+    return (lib.kdecay_scan_saved_states_floats(B, H, N, D, v_code),
+            max(lib.kdecay_scan_workspace_bytes(B, H, N, D, v_code),
+                lib.kdecay_scan_bwd_workspace_bytes(B, H, N, D, v_code)))
+
+
+def _workspace_short_in_capture(dev: torch.device, stream: int, nbytes: int) -> bool:
+    """Whether the stream is being captured and its workspace holds less than
+    nbytes (it cannot grow there)."""
+    ws = _workspaces.get((dev.index, stream))
+    return (nbytes if ws is None else nbytes - ws.numel()) > 0 and torch.cuda.is_current_stream_capturing()
+
+
 class _ScanFn(torch.autograd.Function):
     """The chunked scan with a backward (kdecay_scan_fwd_train / kdecay_scan_bwd).
 
@@ -246,7 +274,8 @@ class _ScanFn(torch.autograd.Function):
     torch autograd through triton_ops.py:240-246, which this replaces on HIP
     tensors.  With sequential=True, y and the final state are then rewritten
     by the sequential kernel (its bits), while the backward uses the states
-    the chunked training forward saved (equal to tolerance).
+    the chunked training forward saved (equal to tolerance).  Head dims the
+    chunked kernels do not take run on the row kernels (_train_sizes).
     """
 
     @staticmethod
@@ -257,20 +286,21 @@ class _ScanFn(torch.autograd.Function):
         o_code = _DTYPE_CODE[out_dtype]
         # The saved V also feeds the backward kernel, whose addressing takes
         # a narrower range of row strides than the forward's.
-        Vk = V if _vector_layout_ok(V) and _bwd_rows_fit(V) else V.contiguous()
+        rows = not chunked_head_dim(D, V.dtype)
+        layout_ok = _row_layout_ok if rows else _train_layout_ok
+        Vk = V if layout_ok(V) else V.contiguous()
         out = torch.empty(Vk.shape, dtype=out_dtype, device=dev) if out_dtype != Vk.dtype else torch.empty_like(Vk)
-        if not _vector_layout_ok(out):
+        if not (_row_layout_ok if rows else _vector_layout_ok)(out):
             out = torch.empty(Vk.shape, dtype=out_dtype, device=dev)
         final = torch.empty((B, H, D), dtype=torch.float32, device=dev)
         lib = _lib.load()
-        nst = lib.kdecay_scan_saved_states_floats(B, H, N, D, v_code)
+        nst, nbytes = _train_sizes(lib, B, H, N, D, v_code, rows)
         states = torch.empty(max(nst, 1), dtype=torch.float32, device=dev)
+        fwd_train = lib.kdecay_scan_fwd_rows_train if rows else lib.kdecay_scan_fwd_train
         with _on_device(dev):
             stream = _stream_ptr(dev)
-            nbytes = max(lib.kdecay_scan_workspace_bytes(B, H, N, D, v_code),
-                         lib.kdecay_scan_bwd_workspace_bytes(B, H, N, D, v_code))
             ws = _workspace(dev, stream, nbytes)
-            rc = lib.kdecay_scan_fwd_train(
+            rc = fwd_train(
                 Vk.data_ptr(), v_code, _lib.strides4(Vk.stride()),
                 out.data_ptr(), o_code, _lib.strides4(out.stride()),
                 lam32.data_ptr(), init32.data_ptr() if init32 is not None else None, final.data_ptr(),
@@ -301,10 +331,11 @@ class _ScanFn(torch.autograd.Function):
         if gy is None:
             gy = torch.zeros_like(Vk)
         gy = gy.to(Vk.dtype)
-        if not (_vector_layout_ok(gy) and _bwd_rows_fit(gy)):
+        rows = not chunked_head_dim(D, Vk.dtype)
+        if not (_row_layout_ok if rows else _train_layout_ok)(gy):
             gy = gy.contiguous()
         dV = torch.empty_like(Vk)
-        if not _vector_layout_ok(dV):
+        if not (_row_layout_ok if rows else _vector_layout_ok)(dV):
             dV = torch.empty(Vk.shape, dtype=Vk.dtype, device=dev)
         dlam = torch.empty(H, dtype=torch.float32, device=dev)
         dinit = torch.empty((B, H, D), dtype=torch.float32, device=dev) if ctx.has_init else None
@@ -312,9 +343,10 @@ class _ScanFn(torch.autograd.Function):
         lib = _lib.load()
         with _on_device(dev):
             stream = _stream_ptr(dev)
-            nbytes = lib.kdecay_scan_bwd_workspace_bytes(B, H, N, D, v_code)
+            nbytes = (lib.kdecay_scan_rows_bwd_workspace_bytes if rows else lib.kdecay_scan_bwd_workspace_bytes)(
+                B, H, N, D, v_code)
             ws = _workspace(dev, stream, nbytes)
-            rc = lib.kdecay_scan_bwd(
+            rc = (lib.kdecay_scan_rows_bwd if rows else lib.kdecay_scan_bwd)(
                 Vk.data_ptr(), v_code, _lib.strides4(Vk.stride()),
                 gy.data_ptr(), _lib.strides4(gy.stride()),
                 dV.data_ptr(), _lib.strides4(dV.stride()),
@@ -457,8 +489,7 @@ def _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, d
     if not _row_vectors_ok(D, V.dtype):
         return False
     nbytes = _fwd_workspace_bytes(lib, B, H, N, D, v_code, rows=True)
-    ws = _workspaces.get((dev.index, stream))
-    if (nbytes if ws is None else nbytes - ws.numel()) > 0 and torch.cuda.is_current_stream_capturing():
+    if _workspace_short_in_capture(dev, stream, nbytes):
         return False
     Vk = V if V.stride(3) == 1 else V.contiguous()
     outk = out if out.stride(3) == 1 else torch.empty(V.shape, dtype=out.dtype, device=dev)
@@ -477,11 +508,23 @@ def _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, d
     return True
 
 
+def _rows_train(V: torch.Tensor) -> bool:
+    """Whether a training pass over V takes the row kernels (see _rows)."""
+    B, H, N, D = V.shape
+    if not _row_vectors_ok(D, V.dtype):
+        return False
+    dev = V.device
+    with _on_device(dev):
+        nbytes = _train_sizes(_lib.load(), B, H, N, D, _DTYPE_CODE[V.dtype], True)[1]
+        return not _workspace_short_in_capture(dev, _stream_ptr(dev), nbytes)
+
+
 def _scan_with_grad(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, algorithm):
     """global_decay_scan when a gradient is required: the chunked training
-    forward and backward under _ScanFn, with differentiable zero-padding of
-    the channels for head dims the kernels do not take, and a differentiable
-    copy into `out` when one is given."""
+    forward and backward under _ScanFn (the row kernels for head dims the
+    chunked ones do not take), with differentiable zero-padding of the channels
+    for head dims neither takes, and a differentiable copy into `out` when one
+    is given."""
     B, H, N, D = V.shape
     dev = V.device
     if algorithm not in ("chunked", "sequential"):
@@ -505,7 +548,7 @@ def _scan_with_grad(lam, V, initial_state, return_final_state, t_offset, out, ou
         y, final = _scan_with_grad(lam, V.float(), initial_state, True, t_offset, None, torch.float32, algorithm)
         y = y.to(torch.float64)
         return (y, final) if return_final_state else y
-    if not chunked_head_dim(D, V.dtype):
+    if not chunked_head_dim(D, V.dtype) and not _rows_train(V):
         Dp = _padded_head_dim(D, V.dtype)
         Vp = torch.nn.functional.pad(V, (0, Dp - D))
         initp = None

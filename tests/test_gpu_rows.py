@@ -1,4 +1,4 @@
-"""The row kernel (kdecay_scan_fwd_rows): head dims and alignments the
+"""The row kernels (kdecay_scan_fwd_rows and its backward): head dims and alignments the
 channel-group kernels refuse, against the oracle and the sequential kernel."""
 from __future__ import annotations
 
@@ -10,6 +10,7 @@ from kilat_amd import _lib
 from kilat_amd.triton_ops import _row_vectors_ok, chunked_head_dim
 from oracle import decay_oracle as O
 from tests.decay_cases import lam_uniform, rel_err
+from tests.test_gpu_grad import check, gpu_grads, oracle_grads
 
 DTYPES = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16, "f64": torch.float64}
 CODES = {"f32": _lib.KDECAY_F32, "bf16": _lib.KDECAY_BF16, "f16": _lib.KDECAY_F16, "f64": _lib.KDECAY_F64}
@@ -157,3 +158,103 @@ def test_rows_under_capture(hip_device, kdecay_lib):
             kilat_amd.triton_global_decay(lam, V[:, :, :1000, :64])
             side.synchronize()
             assert torch.equal(y, ref)
+
+
+def test_rows_backward_rejects_bad_arguments(kdecay_lib):
+    fake = 0x100000
+    ok = (3 * 4096 * 50, 4096 * 50, 50, 1)
+
+    def call(V=fake, D=50, vstr=ok, states=fake, ws=fake, wsb=1 << 30, code=_lib.KDECAY_BF16):
+        return kdecay_lib.kdecay_scan_rows_bwd(V, code, _lib.strides4(vstr), fake, _lib.strides4(ok), fake,
+                                               _lib.strides4(ok), fake, None, states, None, fake, None, 2, 3, 4096, D,
+                                               0, ws, wsb, None)
+
+    assert call(V=None) == _lib.KDECAY_EINVAL
+    assert call(V=fake + 1) == _lib.KDECAY_ELAYOUT
+    assert call(vstr=(3 * 4096 * 100, 4096 * 100, 100, 2)) == _lib.KDECAY_ELAYOUT
+    assert call(D=7) == _lib.KDECAY_ESHAPE
+    assert call(code=_lib.KDECAY_F64) == _lib.KDECAY_EDTYPE
+    assert call(states=None) == _lib.KDECAY_EINVAL
+    assert call(ws=None, wsb=0) == _lib.KDECAY_EWORKSPACE
+    assert call(wsb=4096) == _lib.KDECAY_EWORKSPACE
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname,D", [
+    ("bf16", 8), ("bf16", 9), ("f16", 24), ("bf16", 33), ("f16", 50), ("bf16", 80), ("bf16", 96), ("f16", 127),
+    ("bf16", 136), ("f16", 160), ("bf16", 301), ("f32", 4), ("f32", 5), ("f32", 50), ("f32", 68), ("f32", 100),
+])
+def test_rows_backward_head_dims(hip_device, kdecay_lib, dname, D):
+    """Every kind of row split (whole and shared last vectors, surplus lanes,
+    one to three streams), sequences of one row, around the end of a chunk of
+    4 rows per lane and of several chunks, with a carried state, a final-state
+    gradient and an offset: against fp64 autograd through the oracle."""
+    dtype = DTYPES[dname]
+    g = torch.Generator().manual_seed(1000 + D)
+    lam = lam_uniform(3, 0.5, 0.999, g)
+    nv = -(-D // (16 // torch.empty((), dtype=dtype).element_size()))
+    L = 4 * (64 // -(-nv // -(-nv // 16))) * 4
+    for N, more in ((1, True), (L - 1, False), (L, True), (L + 1, False), (3 * L + 5, True)):
+        V = torch.randn(2, 3, N, D, generator=g).to(dtype)
+        gy = torch.randn(2, 3, N, D, generator=g).to(dtype)
+        init = torch.randn(2, 3, D, generator=g) if more else None
+        gfin = torch.randn(2, 3, D, generator=g) if more else None
+        off = 9 if more else 0
+        dv, dl, di = gpu_grads(lam, V, gy, hip_device, init=init, gfin=gfin, t_offset=off)
+        rdv, rdl, rdi = oracle_grads(lam, V, gy, init=init, gfin=gfin, t_offset=off)
+        check(dv, dl, di, rdv, rdl, rdi, dtype, f"D={D} N={N}")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname,B,H,N,D", [
+    ("bf16", 4, 8, 1001, 96),    # 8 rows per lane, one round
+    ("bf16", 9, 8, 2400, 96),    # 576 chunks of 16 rows per lane
+    ("f16", 8, 9, 3300, 80),     # 648 of them, nine per stream: the wider window
+    ("f32", 10, 12, 900, 50),    # 480 chunks at 16 rows: 8 rows, one round
+    ("f16", 12, 10, 1500, 80),   # several rounds
+    ("f32", 2, 3, 3000, 20),     # 4 rows per lane, chains of a few tens of chunks
+    ("bf16", 1, 1, 9000, 100),   # a longer chain: the wide window
+    ("bf16", 20, 12, 60, 48),    # 240 streams of one chunk
+])
+def test_rows_backward_grids(hip_device, kdecay_lib, dname, B, H, N, D):
+    """From the projection layout, V and the gradient alike, against the
+    channel-group kernels on zero-padded rows (padding changes no value; those
+    kernels have their own tests against the oracle); the same bits on every
+    run; gradients laid out like V."""
+    dtype = DTYPES[dname]
+    g = torch.Generator().manual_seed(1100 + D)
+    lam = lam_uniform(H, 0.5, 0.999, g)
+    V = torch.randn(B, N, H, D, generator=g).to(dtype).transpose(1, 2)
+    gy = torch.randn(B, N, H, D, generator=g).to(dtype).transpose(1, 2)
+    Dp = -(-D // 64) * 64
+    V_p = torch.nn.functional.pad(V, (0, Dp - D)).to(hip_device).requires_grad_()
+    lam_p = lam.to(hip_device).requires_grad_()
+    y_p = kilat_amd.triton_global_decay(lam_p, V_p)
+    rdv, rdl = torch.autograd.grad(y_p, (V_p, lam_p), torch.nn.functional.pad(gy, (0, Dp - D)).to(hip_device))
+    rdv, rdl, y_p = rdv[..., :D].double().cpu(), rdl.cpu(), y_p.detach()[..., :D]
+    first = None
+    for _ in range(2):
+        lam_d = lam.to(hip_device).requires_grad_()
+        V_d = V.transpose(1, 2).to(hip_device).transpose(1, 2).requires_grad_()
+        y = kilat_amd.triton_global_decay(lam_d, V_d)
+        dv, dl = torch.autograd.grad(y, (V_d, lam_d), gy.transpose(1, 2).to(hip_device).transpose(1, 2))
+        assert dv.stride() == V_d.stride() == y.stride()
+        assert rel_err(y.detach(), y_p) <= TOL[dtype]
+        check(dv.cpu(), dl.cpu(), None, rdv, rdl, None, dtype, f"grid D={D}")
+        assert first is None or (torch.equal(first[0], dv) and torch.equal(first[1], dl))
+        first = dv, dl
+
+
+@pytest.mark.gpu
+def test_rows_backward_infinite_gradient_stays_in_its_channel(hip_device, kdecay_lib):
+    """An infinite gradient at the last row: every earlier row of that channel
+    is infinite (never NaN from rows past the end), the others are finite, also
+    where a row's last vector repeats the channel."""
+    for D, c in ((48, 0), (50, 45)):
+        lam = torch.full((2,), 0.99, device=hip_device, requires_grad=True)
+        V = torch.randn(1, 2, 77, D, device=hip_device).to(torch.bfloat16).requires_grad_()
+        gy = torch.randn(1, 2, 77, D, device=hip_device).to(torch.bfloat16)
+        gy[:, :, -1, c] = float("inf")
+        dv, = torch.autograd.grad(kilat_amd.triton_global_decay(lam, V), V, gy)
+        assert torch.isposinf(dv[..., c]).all()
+        assert torch.isfinite(dv[..., :c]).all() and torch.isfinite(dv[..., c + 1:]).all()

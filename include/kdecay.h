@@ -122,6 +122,12 @@ int kdecay_scan_fwd(const void* V, int v_dtype, const int64_t* v_strides,
 size_t kdecay_scan_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t D,
                                    int v_dtype);
 
+/* The least kdecay_scan_fwd accepts for this shape, at most the above.  With a
+ * workspace between the two it splits the sequences as kdecay_scan_fwd_train
+ * does (results equal up to rounding). */
+size_t kdecay_scan_workspace_least_bytes(int64_t B, int64_t H, int64_t N,
+                                         int64_t D, int v_dtype);
+
 /*
  * kdecay_scan_fwd for every head dim and alignment: the same arguments,
  * results, workspace rules and error handling (its workspace is

@@ -32,6 +32,7 @@ KDECAY_NOALLOC_WORKSPACE_BYTES = 8 << 20  # include/kdecay.h
 EXPORTS = (
     "kdecay_scan_fwd",
     "kdecay_scan_workspace_bytes",
+    "kdecay_scan_workspace_least_bytes",
     "kdecay_scan_fwd_rows",
     "kdecay_scan_rows_workspace_bytes",
     "kdecay_scan_fwd_rows_train",
@@ -81,6 +82,8 @@ def load() -> ctypes.CDLL:
     ]
     lib.kdecay_scan_workspace_bytes.restype = ctypes.c_size_t
     lib.kdecay_scan_workspace_bytes.argtypes = [_c_i64, _c_i64, _c_i64, _c_i64, ctypes.c_int]
+    lib.kdecay_scan_workspace_least_bytes.restype = ctypes.c_size_t
+    lib.kdecay_scan_workspace_least_bytes.argtypes = lib.kdecay_scan_workspace_bytes.argtypes
     lib.kdecay_scan_fwd_rows.restype = ctypes.c_int
     lib.kdecay_scan_fwd_rows.argtypes = lib.kdecay_scan_fwd.argtypes
     lib.kdecay_scan_rows_workspace_bytes.restype = ctypes.c_size_t

@@ -1282,7 +1282,54 @@ constexpr int64_t kSixWideLo = 1024;
 constexpr int kNWLong = 8;
 constexpr int64_t kLongChain = 64;
 
-ChunkShape chunk_shape(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype) {
+// Short sequences: the smallest chunk that holds the whole sequence, of 4 rows x
+// 1 wavefront, 8 x 1, 4 x 4 or 8 x 4 (32, 64, 128 and 256 rows of a 128-byte
+// group).  In a chunk of 512 the lanes past the end only repeat row N-1, and a
+// call of many short prompts runs that many more workgroups' worth of rounds.
+// Measured (bf16 D=64 H=12, projection layout, us, 512-row chunks in batch
+// slices / this; a copy of the bytes): B=1024 N=32 82.3 / 22.2 (19.4), B=512
+// N=64 70.6 / 21.7 (19.4), B=512 N=100 73.6 / 31.9 (30.3), B=256 N=128 34.1 /
+// 21.8 (19.4), B=256 N=200 42.3 / 32.8 (30.3), B=192 N=256 30.5 / 30.8 (29.1);
+// few sequences: B=64 N=100 9.5 / 6.9, B=32 N=200 8.9 / 6.8, B=8 N=60 6.0 / 5.7.
+//
+// Sequences that fill at most three quarters of their 512-row chunks (N in
+// (256, 384], (512, 768], (1024, 1152]): 12 rows per lane, 384-row chunks, as
+// many per stream.  Measured (us, 512-row chunks, in slices where those applied
+// / 384-row; a copy): N=300 B=30 10.4 / 8.7 (5.3), B=128 29.4 / 26.6 (22.7),
+// B=200 53.5 / 38.8 (35.5); N=520 B=64 28.0 / 23.9 (19.7); N=600 B=30 14.6 /
+// 12.3, B=80 35.9 / 32.3 (28.4), B=100 62.5 / 39.4 (35.5); N=700 B=40 19.3 /
+// 16.6 (16.6), B=64 31.1 / 28.1; N=1100 B=20 16.1 / 13.8 (13.0), B=40 31.8 /
+// 29.2, B=60 47.5 / 41.5 (39.1).  At five sixths (N=1280) the slices of 512 win
+// (B=40 29.3 against 31.2 of 256-row chunks).  Small grids keep their 8-row
+// chunks (N=700 B=8 7.4 / 8.5; with 2 chunks per stream to 560: H=7 N=655 B=33,
+// 462 chunks, 10.4 / 11.1) unless one 384-row chunk holds the sequence
+// (N=300 B=16 9.2 / 7.3, B=8 7.8 / 7.1), and wide heads their six-per-CU grid
+// (bf16 D=256 H=1 B=216 N=611 28.8 / 31.2).  256- and 192-row chunks were up to 13%
+// faster than 384 on grids of several rounds (N=520 B=64 20.7), but need more
+// look-back words than the 512-row chunks did: a workspace sized before could be
+// too small.  Not when the forward saves states: its lanes' ends then have to
+// meet the backward's chunk starts, which are no multiples of 12 rows.
+constexpr int kRTiny = 4;
+constexpr int kRFit = 12;
+constexpr int64_t kFitGrid2 = 560;
+
+bool fit_rows(int64_t N, int64_t gw) {
+  const int64_t l16 = kNW * gw * kR, l12 = kNW * gw * kRFit;
+  const int64_t p16 = (N + l16 - 1) / l16 * l16, p12 = (N + l12 - 1) / l12 * l12;
+  return 3 * p16 >= 4 * p12;
+}
+
+// Row groups per wavefront of the forward's streams.
+int64_t row_groups(int v_dtype, int64_t D) { return 64 / (group_width(v_dtype, D) * elem_size(v_dtype) / 16); }
+
+// saves: the launch saves the backward's states (more than one backward chunk
+// per stream).
+ChunkShape chunk_shape(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves) {
+  const int64_t gw = row_groups(v_dtype, D);
+  if (N <= gw * kRTiny) return ChunkShape{kRTiny, 1};
+  if (N <= gw * kRSmall) return ChunkShape{kRSmall, 1};
+  if (N <= gw * kRTiny * kNWSmall) return ChunkShape{kRTiny, kNWSmall};
+  if (N <= gw * kRSmall * kNWSmall) return ChunkShape{kRSmall, kNWSmall};
   const int64_t L = chunk_rows(v_dtype, D, ChunkShape{kR, kNW});
   const int64_t ng = D / group_width(v_dtype, D);
   const int64_t nstream = B * H * ng;
@@ -1290,14 +1337,16 @@ ChunkShape chunk_shape(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype) 
   const int64_t grid = chain * nstream;
   const int64_t lim = chain == 1 ? kSmallGrid1 : chain == 2 ? kSmallGrid2 : kSmallGrid;
   const bool full = group_width(v_dtype, D) * elem_size(v_dtype) == 128;
+  const bool wide = full && ng >= kSixWideGroups && chain <= kSixWideChain && grid >= kSixWideLo;
+  if (!saves && !wide && fit_rows(N, gw) && (chain == 1 || grid > (chain == 2 ? kFitGrid2 : kSmallGrid)))
+    return ChunkShape{kRFit, kNW};
   if (grid <= lim) {
     const int64_t chain8 = (N + L / 2 - 1) / (L / 2);  // chunks per stream at 8 rows per lane
     return full && chain8 >= kLongChain ? ChunkShape{kRSmall, kNWLong} : ChunkShape{kRSmall, kNWSmall};
   }
   if (full && chain <= kSixChain && grid > (ng > 1 ? kSixLoGroups : kSixLo) && grid <= kSixHi)
     return ChunkShape{kRSmall, kNWSmall, true};
-  if (full && ng >= kSixWideGroups && chain <= kSixWideChain && grid >= kSixWideLo)
-    return ChunkShape{kRSmall, kNWSmall, true};
+  if (wide) return ChunkShape{kRSmall, kNWSmall, true};
   return ChunkShape{kR, kNW};
 }
 
@@ -1337,9 +1386,12 @@ constexpr int64_t kSliceRound = 1024;
 constexpr int64_t kSliceCUs = 256;
 constexpr int64_t kSliceChain = 8;
 constexpr int64_t kSliceMax = 8;
-int64_t fwd_slices(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype) {
+// Only sequences that run in 512-row chunks (chunk_shape).
+int64_t fwd_slices(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves) {
   const int64_t DG = group_width(v_dtype, D);
   if (B < 2 || DG != D || DG * elem_size(v_dtype) != 128) return 1;
+  const int64_t gw = row_groups(v_dtype, D);
+  if (N <= gw * kRSmall * kNWSmall || (!saves && fit_rows(N, gw))) return 1;
   const int64_t L = chunk_rows(v_dtype, D, ChunkShape{kR, kNW});
   const int64_t chain = (N + L - 1) / L;
   const int64_t per_b = H * chain;  // 512-row chunks of one batch element
@@ -1375,8 +1427,20 @@ int launch_chunked(const ScanArgs& a, int64_t grid, hipStream_t s, bool six = fa
   // the unrolled, branch-free power (B=8 N=1024 H=6 D=64 bf16: 7.07 -> 6.85
   // us); for large grids the loop form is cheaper (B=8 N=4096 H=12 D=64:
   // 18.36 vs 18.74 us with the unrolled one).  Same values either way.
-  constexpr bool FZ = R == kRSmall && NW == kNWSmall;
-  if constexpr (FZ) {
+  constexpr bool FZ = R <= kRSmall;
+  if constexpr (R == kRTiny || NW == 1) {
+    // One chunk per stream (chunk_shape): no look-back.
+    hipLaunchKernelGGL((scan_chunked<TI, TO, LPR, R, NW, 1, WPE, FZ, false>), dim3((unsigned)grid), dim3(NW * 64), 0, s,
+                       a);
+  } else if constexpr (R == kRFit) {
+    // Stores throttled (THR) where the grid nearly fills its one round (five
+    // workgroups per CU): N=700 B=40 (960 chunks) 18.7 -> 16.6 us; at 720 (N=600
+    // B=30) 12.3 -> 12.6, in two rounds (N=700 B=64) 28.1 -> 30.4.
+    const int64_t cus = cu_count();
+    auto* const k = grid > 3 * cus && grid <= 5 * cus ? scan_chunked<TI, TO, LPR, R, NW, 1, WPE, FZ, true>
+                                                      : scan_chunked<TI, TO, LPR, R, NW, 1, WPE, FZ, false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(NW * 64), 0, s, a);
+  } else if constexpr (FZ) {
     if constexpr (LPR == 8) {  // full 128-byte channel groups
       if (six) {  // chunk_shape's 8-row grid, six workgroups per CU (two rounds at most, except wide heads)
         hipLaunchKernelGGL((scan_chunked<TI, TO, LPR, R, NW, 1, 6, FZ, false>), dim3((unsigned)grid), dim3(NW * 64), 0,
@@ -1466,6 +1530,10 @@ int dispatch_dg(const ScanArgs& a, int64_t DG, int64_t grid, hipStream_t s, Chun
     return fail(KDECAY_ESHAPE, "unsupported channel group %lld", (long long)DG);
   }
   if (c.R == kRSmall && c.NW == kNWSmall) return dispatch_dg_r<TI, TO, kRSmall, kNWSmall>(a, DG, grid, s, c.six);
+  if (c.R == kRTiny && c.NW == 1) return dispatch_dg_r<TI, TO, kRTiny, 1>(a, DG, grid, s, false);
+  if (c.R == kRSmall && c.NW == 1) return dispatch_dg_r<TI, TO, kRSmall, 1>(a, DG, grid, s, false);
+  if (c.R == kRTiny) return dispatch_dg_r<TI, TO, kRTiny, kNWSmall>(a, DG, grid, s, false);
+  if (c.R == kRFit) return dispatch_dg_r<TI, TO, kRFit, kNW>(a, DG, grid, s, false);
   return dispatch_dg_r<TI, TO, kR, kNW>(a, DG, grid, s, false);
 }
 
@@ -1756,15 +1824,37 @@ uint32_t kdecay_debug_fastdiv(uint32_t n, uint32_t d, int want_mod) {
   return want_mod ? f.mod(n) : f.div(n);
 }
 
+// How the forward runs a shape, with or without saved states.
+struct FwdPlan {
+  int64_t nslice;    // launches, over balanced slices of the batch
+  ChunkShape shape;
+  int64_t L, nchunk;  // rows of a chunk, chunks per stream
+  size_t need;       // workspace bytes: slices run one after another on it, so the largest one's
+};
+
+static FwdPlan fwd_plan(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves) {
+  FwdPlan p;
+  p.nslice = fwd_slices(B, H, N, D, v_dtype, saves);
+  p.shape = p.nslice > 1 ? ChunkShape{kR, kNW} : chunk_shape(B, H, N, D, v_dtype, saves);
+  p.L = chunk_rows(v_dtype, D, p.shape);
+  p.nchunk = (N + p.L - 1) / p.L;
+  const int64_t Bs = (B + p.nslice - 1) / p.nslice;
+  p.need = p.nchunk <= 1 ? 0 : kHeaderBytes + (size_t)(Bs * H * p.nchunk * D) * sizeof(u64);
+  return p;
+}
+
 size_t kdecay_scan_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype) {
   if (B <= 0 || H <= 0 || N <= 0 || !fwd_dtype_ok(v_dtype) || !head_dim_ok(v_dtype, D)) return 0;
-  const int64_t n = fwd_slices(B, H, N, D, v_dtype);
-  // Batch slices run one after another on the workspace: the largest one's.
-  const int64_t Bs = (B + n - 1) / n;
-  const int64_t L = chunk_rows(v_dtype, D, n > 1 ? ChunkShape{kR, kNW} : chunk_shape(B, H, N, D, v_dtype));
-  const int64_t nchunk = (N + L - 1) / L;
-  if (nchunk <= 1) return 0;
-  return kHeaderBytes + (size_t)(Bs * H * nchunk * D) * sizeof(u64);
+  const size_t plain = fwd_plan(B, H, N, D, v_dtype, false).need;
+  const size_t saving = fwd_plan(B, H, N, D, v_dtype, true).need;  // kdecay_scan_fwd_train's
+  return plain > saving ? plain : saving;
+}
+
+// The shapes of a saving launch need no more than any other (chunk_shape's
+// 384-row chunks run in one launch where 512-row ones run in batch slices).
+size_t kdecay_scan_workspace_least_bytes(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype) {
+  if (B <= 0 || H <= 0 || N <= 0 || !fwd_dtype_ok(v_dtype) || !head_dim_ok(v_dtype, D)) return 0;
+  return fwd_plan(B, H, N, D, v_dtype, true).need;
 }
 
 static int scan_fwd_impl(const void* V, int v_dtype, const int64_t* v_strides, void* out, int out_dtype,
@@ -1791,32 +1881,35 @@ static int scan_fwd_impl(const void* V, int v_dtype, const int64_t* v_strides, v
   }
 
   const int64_t DG = group_width(v_dtype, D);
+  // The training forward's saved states follow the whole batch's backward
+  // chunks, and batch 0's workgroups write the per-row terms once.
+  const int64_t state_rows = states ? bwd_chunk_rows(B, H, N, D, v_dtype) : N;
+  const int64_t nsaved = (N + state_rows - 1) / state_rows;
+  float* const saved = nsaved > 1 ? states : nullptr;
+  float2* const rowtab = saved ? reinterpret_cast<float2*>(saved + B * H * D * nsaved) : nullptr;
+  // A workspace of less than kdecay_scan_workspace_bytes, but enough for a
+  // saving launch's shapes, takes those.
+  FwdPlan plan = fwd_plan(B, H, N, D, v_dtype, saved != nullptr);
+  if (workspace_bytes < plan.need && !saved) plan = fwd_plan(B, H, N, D, v_dtype, true);
+  const int64_t L = plan.L, nchunk = plan.nchunk, nslice = plan.nslice;
+  const bool multi = nchunk > 1;
   {
-    const int64_t L = chunk_rows(v_dtype, D, chunk_shape(B, H, N, D, v_dtype));
-    const int64_t nchunk = (N + L - 1) / L, nstream = B * H * (D / DG), grid = nchunk * nstream;
+    const int64_t nstream = B * H * (D / DG), grid = nchunk * nstream;
     if (grid > 0x7fffffffLL || nchunk > 0x7fffffffLL || nstream > 0x7fffffffLL)
       return fail(KDECAY_EINVAL, "problem too large (%lld chunks)", (long long)grid);
   }
-  const size_t need = kdecay_scan_workspace_bytes(B, H, N, D, v_dtype);
+  // One wavefront holds at most 8 rows per row group, less than any backward
+  // chunk (4 wavefronts): it saves nothing (ChunkScan::scan_chunk).
+  if (plan.shape.NW == 1 && saved) return fail(KDECAY_EINVAL, "no saving kernel of one wavefront");
+  const size_t need = plan.need;
   if (need && (!workspace || workspace_bytes < need))
     return fail(KDECAY_EWORKSPACE, "workspace of %zu bytes required, %zu given", need, workspace_bytes);
   if (need && ((uintptr_t)workspace & 255u)) return fail(KDECAY_EWORKSPACE, "workspace must be 256-byte aligned");
 
-  // The training forward's saved states follow the whole batch's backward
-  // chunks, and batch 0's workgroups write the per-row terms once.
-  const int64_t state_rows = bwd_chunk_rows(B, H, N, D, v_dtype);
-  const int64_t nsaved = (N + state_rows - 1) / state_rows;
-  float* const saved = nsaved > 1 ? states : nullptr;
-  float2* const rowtab = saved ? reinterpret_cast<float2*>(saved + B * H * D * nsaved) : nullptr;
-  const int64_t nslice = fwd_slices(B, H, N, D, v_dtype);
   for (int64_t i = 0; i < nslice; ++i) {
     const int64_t b0 = B * i / nslice, Bs = B * (i + 1) / nslice - b0;
-    const ChunkShape shape = nslice > 1 ? ChunkShape{kR, kNW} : chunk_shape(B, H, N, D, v_dtype);
-    const int64_t L = chunk_rows(v_dtype, D, shape);
-    const int64_t nchunk = (N + L - 1) / L;
     const int64_t nstream = Bs * H * (D / DG);
     const int64_t grid = nchunk * nstream;
-    const bool multi = nchunk > 1;
 
     ScanArgs a;
     a.V = static_cast<const char*>(V) + b0 * v_strides[0] * elem_size(v_dtype);
@@ -1849,15 +1942,15 @@ static int scan_fwd_impl(const void* V, int v_dtype, const int64_t* v_strides, v
     a.rowtab = i == 0 ? rowtab : nullptr;
 
     if (v_dtype == KDECAY_F32)
-      rc = dispatch_dg<float, float>(a, DG, grid, s, shape);
+      rc = dispatch_dg<float, float>(a, DG, grid, s, plan.shape);
     else if (v_dtype == KDECAY_F64)
-      rc = dispatch_dg<double, double>(a, DG, grid, s, shape);
+      rc = dispatch_dg<double, double>(a, DG, grid, s, plan.shape);
     else if (v_dtype == KDECAY_BF16)
-      rc = out_dtype == KDECAY_BF16 ? dispatch_dg<__bf16, __bf16>(a, DG, grid, s, shape)
-                                    : dispatch_dg<__bf16, float>(a, DG, grid, s, shape);
+      rc = out_dtype == KDECAY_BF16 ? dispatch_dg<__bf16, __bf16>(a, DG, grid, s, plan.shape)
+                                    : dispatch_dg<__bf16, float>(a, DG, grid, s, plan.shape);
     else
-      rc = out_dtype == KDECAY_F16 ? dispatch_dg<_Float16, _Float16>(a, DG, grid, s, shape)
-                                   : dispatch_dg<_Float16, float>(a, DG, grid, s, shape);
+      rc = out_dtype == KDECAY_F16 ? dispatch_dg<_Float16, _Float16>(a, DG, grid, s, plan.shape)
+                                   : dispatch_dg<_Float16, float>(a, DG, grid, s, plan.shape);
     if (rc) return rc;
   }
   return 0;

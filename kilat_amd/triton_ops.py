@@ -437,8 +437,12 @@ def global_decay_scan(
             _chunked(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev)
         elif _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev):
             pass
-        elif chunked_head_dim(D, V.dtype):
-            _chunked(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev)
+        elif chunked_head_dim(D, V.dtype):  # through contiguous copies
+            Vk = V if _vector_layout_ok(V) else V.contiguous()
+            outk = out if _vector_layout_ok(out) else torch.empty(V.shape, dtype=out.dtype, device=dev)
+            _chunked(lib, Vk, v_code, outk, o_code, lam32, init32, final, t_offset, stream, dev)
+            if outk is not out:
+                out.copy_(outk)
         else:  # zero channels up to a head dim the chunked kernels take
             Dp = _padded_head_dim(D, V.dtype)
             Vp = V.new_zeros((B, H, N, Dp))
@@ -459,24 +463,21 @@ def global_decay_scan(
 
 
 def _chunked(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev) -> None:
-    """kdecay_scan_fwd on V into out (through contiguous copies where the
-    layout is not one the vector kernel takes)."""
+    """kdecay_scan_fwd on V into out, in layouts the vector kernel takes."""
     B, H, N, D = V.shape
-    Vk = V if _vector_layout_ok(V) else V.contiguous()
-    outk = out if _vector_layout_ok(out) else torch.empty(V.shape, dtype=out.dtype, device=dev)
     nbytes = _fwd_workspace_bytes(lib, B, H, N, D, v_code)
+    if nbytes and _workspace_short_in_capture(dev, stream, nbytes):
+        nbytes = lib.kdecay_scan_workspace_least_bytes(B, H, N, D, v_code)
     ws = _workspace(dev, stream, nbytes)
     rc = lib.kdecay_scan_fwd(
-        Vk.data_ptr(), v_code, _lib.strides4(Vk.stride()),
-        outk.data_ptr(), o_code, _lib.strides4(outk.stride()),
+        V.data_ptr(), v_code, _lib.strides4(V.stride()),
+        out.data_ptr(), o_code, _lib.strides4(out.stride()),
         lam32.data_ptr(), init32.data_ptr() if init32 is not None else None,
         final.data_ptr() if final is not None else None, B, H, N, D, int(t_offset),
         ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0,
         stream,
     )
     _lib.check(rc, "kdecay_scan_fwd")
-    if outk is not out:
-        out.copy_(outk)
 
 
 def _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev) -> bool:

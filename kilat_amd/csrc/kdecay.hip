@@ -1172,10 +1172,13 @@ int64_t group_width(int v_dtype, int64_t D) {
 // rounds at 128 bytes; chains of 16 at 256 rows) 65.5 / 61.0; B=4 N=4096
 // H=12 30.8 / 29.9; but B=1 N=65536 H=16 (chains of 256) 145.7 / 165.9 and
 // B=8 N=1024 H=6 (a small grid, 128-row chunks at 128 bytes) 12.6 / 13.6.
+// Sequences of up to 128 rows have smaller chunks of 128-byte groups
+// (bwd_shape).
+constexpr int64_t kWideShort = 128;
 constexpr int64_t kWideChain = 32;  // chunks of 256 rows per stream, at most
 constexpr int64_t kWideGrid = 512;  // chunks of 256 rows in all, at least
 int64_t bwd_group_width(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype) {
-  if (elem_size(v_dtype) == 2 && D % 128 == 0) {
+  if (elem_size(v_dtype) == 2 && D % 128 == 0 && N > kWideShort) {
     const int64_t chain = (N + 255) / 256;
     if (chain <= kWideChain && chain * B * H * (D / 128) >= kWideGrid) return 128;
   }
@@ -1283,40 +1286,80 @@ constexpr int kNWLong = 8;
 constexpr int64_t kLongChain = 64;
 
 // Short sequences: the smallest chunk that holds the whole sequence, of 4 rows x
-// 1 wavefront, 8 x 1, 4 x 4 or 8 x 4 (32, 64, 128 and 256 rows of a 128-byte
-// group).  In a chunk of 512 the lanes past the end only repeat row N-1, and a
-// call of many short prompts runs that many more workgroups' worth of rounds.
-// Measured (bf16 D=64 H=12, projection layout, us, 512-row chunks in batch
-// slices / this; a copy of the bytes): B=1024 N=32 82.3 / 22.2 (19.4), B=512
-// N=64 70.6 / 21.7 (19.4), B=512 N=100 73.6 / 31.9 (30.3), B=256 N=128 34.1 /
-// 21.8 (19.4), B=256 N=200 42.3 / 32.8 (30.3), B=192 N=256 30.5 / 30.8 (29.1);
-// few sequences: B=64 N=100 9.5 / 6.9, B=32 N=200 8.9 / 6.8, B=8 N=60 6.0 / 5.7.
+// 1 wavefront, 8 x 1, 4 x 4 or (128-byte groups) 8 x 4: 32, 64, 128 and 256 rows
+// of a 128-byte group.  In a chunk of 512 the lanes past the end only repeat row
+// N-1, and a call of many short prompts runs that many more workgroups' worth of
+// rounds.  Measured (bf16 D=64 H=12, projection layout, us, 512-row chunks in
+// batch slices / this; a copy of the bytes): B=1024 N=32 82.3 / 22.2 (19.4),
+// B=512 N=64 70.6 / 21.7 (19.4), B=512 N=100 73.6 / 31.9 (30.3), B=256 N=128 34.1
+// / 21.8 (19.4), B=256 N=200 42.3 / 32.8 (30.3), B=192 N=256 30.5 / 30.8 (29.1);
+// few sequences: B=64 N=100 9.5 / 6.9, B=32 N=200 8.9 / 6.8, B=8 N=60 6.0 / 5.7;
+// D=16 B=400 N=60 46.1 / 14.8, N=130 41.8 / 28.7, D=32 B=400 N=100 37.8 / 22.3,
+// N=200 43.7 / 36.7.  Narrow groups keep 16 rows x 4 wavefronts beyond 4 x 4
+// (contiguous D=16 H=4 B=628 N=719: 56.3, 8 x 4 68.5).
 //
-// Sequences that fill at most three quarters of their 512-row chunks (N in
-// (256, 384], (512, 768], (1024, 1152]): 12 rows per lane, 384-row chunks, as
-// many per stream.  Measured (us, 512-row chunks, in slices where those applied
-// / 384-row; a copy): N=300 B=30 10.4 / 8.7 (5.3), B=128 29.4 / 26.6 (22.7),
-// B=200 53.5 / 38.8 (35.5); N=520 B=64 28.0 / 23.9 (19.7); N=600 B=30 14.6 /
-// 12.3, B=80 35.9 / 32.3 (28.4), B=100 62.5 / 39.4 (35.5); N=700 B=40 19.3 /
-// 16.6 (16.6), B=64 31.1 / 28.1; N=1100 B=20 16.1 / 13.8 (13.0), B=40 31.8 /
-// 29.2, B=60 47.5 / 41.5 (39.1).  At five sixths (N=1280) the slices of 512 win
-// (B=40 29.3 against 31.2 of 256-row chunks).  Small grids keep their 8-row
-// chunks (N=700 B=8 7.4 / 8.5; with 2 chunks per stream to 560: H=7 N=655 B=33,
-// 462 chunks, 10.4 / 11.1) unless one 384-row chunk holds the sequence
-// (N=300 B=16 9.2 / 7.3, B=8 7.8 / 7.1), and wide heads their six-per-CU grid
-// (bf16 D=256 H=1 B=216 N=611 28.8 / 31.2).  256- and 192-row chunks were up to 13%
-// faster than 384 on grids of several rounds (N=520 B=64 20.7), but need more
-// look-back words than the 512-row chunks did: a workspace sized before could be
-// too small.  Not when the forward saves states: its lanes' ends then have to
-// meet the backward's chunk starts, which are no multiples of 12 rows.
+// Sequences of a 128-byte group that leave much of their 512-row chunks empty
+// run in 384-row chunks of 12 rows per lane, as many per stream.  Measured (us,
+// 512-row chunks, in slices where those applied / 384-row; a copy): N=300 B=30
+// 10.5 / 8.7 (5.3), B=80 16.9 / 15.2, B=200 53.0 / 38.1 (35.5); N=360 B=30 10.3 /
+// 9.3, B=80 18.8 / 19.9, B=200 52.6 / 45.1; N=600 B=30 14.7 / 12.4, B=60 29.2 /
+// 25.5, B=128 59.4 / 50.0 (45.5); N=700 B=42 19.5 / 17.3, B=128 60.9 / 54.6; N=768
+// B=60 27.7 / 30.9; N=1100 B=20 16.1 / 13.8, B=64 65.6 / 43.9 (41.7); N=1152 B=28
+// 20.5 / 18.6, B=40 28.0 / 29.0, B=64 56.6 / 44.1; N=1280 (five sixths) B=40 29.3
+// / 31.2.  One chunk per stream in two slices that fill their workgroup slots
+// gains nothing (B=128, two slices of 768: N=270 23.3 / 25.1, N=300 26.7 / 26.4, N=340
+// 26.0 / 29.5), nor do small grids, which keep 8 rows (H=13 B=1 N=331 D=128 6.7 /
+// 7.8; N=700 B=8 7.4 / 8.5; two chunks per stream to 560: H=7 N=655 B=33 10.4 /
+// 11.1), and wide heads (D=256 H=1 B=216 N=611 28.8 / 31.2).  256- and 192-row
+// chunks were up to 13% faster than 384 on grids of several rounds (N=520 B=64
+// 20.7 against 23.9), but need more look-back words than the 512-row chunks did:
+// a workspace sized before could be too small.  Not when the forward saves
+// states: its lanes' ends then have to meet the backward's chunk starts, which
+// are no multiples of 12 rows.
 constexpr int kRTiny = 4;
 constexpr int kRFit = 12;
 constexpr int64_t kFitGrid2 = 560;
 
-bool fit_rows(int64_t N, int64_t gw) {
-  const int64_t l16 = kNW * gw * kR, l12 = kNW * gw * kRFit;
-  const int64_t p16 = (N + l16 - 1) / l16 * l16, p12 = (N + l12 - 1) / l12 * l12;
-  return 3 * p16 >= 4 * p12;
+constexpr int64_t kSliceRound = 1024;
+constexpr int64_t kSliceCUs = 256;
+constexpr int64_t kSliceChain = 8;
+constexpr int64_t kSliceMax = 8;
+
+// Whether 512-row chunks run as batch slices (fwd_slices): per_b of them per
+// batch element, chain per stream, ng groups per head.
+bool sliceable(int64_t B, int64_t chain, int64_t per_b, int64_t ng) {
+  return B >= 2 && ng == 1 && chain <= kSliceChain && per_b <= kSliceRound && B * per_b > kSliceRound &&
+         (B + kSliceRound / per_b - 1) / (kSliceRound / per_b) <= kSliceMax;
+}
+
+// The number of slices, and whether they fill nine tenths of their workgroup slots.
+int64_t slice_count(int64_t B, int64_t per_b, bool* fill) {
+  const int64_t b_max = kSliceRound / per_b;
+  const int64_t fewest = (B + b_max - 1) / b_max;
+  int64_t best = fewest, best_rounds = 0;
+  for (int64_t n = fewest; n <= fewest + 2 && n <= B && n <= kSliceMax; ++n) {
+    const int64_t rounds = n * (((B + n - 1) / n * per_b + kSliceCUs - 1) / kSliceCUs);
+    if (n == fewest || rounds < best_rounds) best = n, best_rounds = rounds;
+  }
+  const int64_t chunks = (B + best - 1) / best * per_b;
+  const int64_t slots = (chunks + kSliceCUs - 1) / kSliceCUs * kSliceCUs;
+  *fill = 10 * chunks >= 9 * slots;
+  return best;
+}
+
+// N rows in `chain` chunks of 512 (gw row groups per wavefront: 8), `grid` of
+// them in all, `slices`: run as batch slices otherwise.
+bool fit_rows(int64_t B, int64_t N, int64_t gw, int64_t chain, int64_t grid, bool slices) {
+  const int64_t l12 = kNW * gw * kRFit, p16 = chain * kNW * gw * kR;
+  if ((N + l12 - 1) / l12 != chain) return false;
+  if (chain >= 3) return 4 * N <= 3 * p16 && grid > kSmallGrid;
+  if (chain == 2) return 100 * N <= 72 * p16 && grid > kFitGrid2;
+  if (grid <= kSmallGrid1 || 100 * N > 71 * p16) return false;
+  if (slices) {
+    bool fill;
+    return slice_count(B, grid / B, &fill) > 2 || !fill;
+  }
+  return grid <= 720 || 10 * N <= 6 * p16 || grid > 1024;
 }
 
 // Row groups per wavefront of the forward's streams.
@@ -1326,19 +1369,19 @@ int64_t row_groups(int v_dtype, int64_t D) { return 64 / (group_width(v_dtype, D
 // per stream).
 ChunkShape chunk_shape(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves) {
   const int64_t gw = row_groups(v_dtype, D);
+  const bool full = group_width(v_dtype, D) * elem_size(v_dtype) == 128;
   if (N <= gw * kRTiny) return ChunkShape{kRTiny, 1};
   if (N <= gw * kRSmall) return ChunkShape{kRSmall, 1};
   if (N <= gw * kRTiny * kNWSmall) return ChunkShape{kRTiny, kNWSmall};
-  if (N <= gw * kRSmall * kNWSmall) return ChunkShape{kRSmall, kNWSmall};
+  if (full && N <= gw * kRSmall * kNWSmall) return ChunkShape{kRSmall, kNWSmall};
   const int64_t L = chunk_rows(v_dtype, D, ChunkShape{kR, kNW});
   const int64_t ng = D / group_width(v_dtype, D);
   const int64_t nstream = B * H * ng;
   const int64_t chain = (N + L - 1) / L;
   const int64_t grid = chain * nstream;
   const int64_t lim = chain == 1 ? kSmallGrid1 : chain == 2 ? kSmallGrid2 : kSmallGrid;
-  const bool full = group_width(v_dtype, D) * elem_size(v_dtype) == 128;
   const bool wide = full && ng >= kSixWideGroups && chain <= kSixWideChain && grid >= kSixWideLo;
-  if (!saves && !wide && fit_rows(N, gw) && (chain == 1 || grid > (chain == 2 ? kFitGrid2 : kSmallGrid)))
+  if (full && !saves && !wide && fit_rows(B, N, gw, chain, grid, sliceable(B, chain, H * chain, ng)))
     return ChunkShape{kRFit, kNW};
   if (grid <= lim) {
     const int64_t chain8 = (N + L / 2 - 1) / (L / 2);  // chunks per stream at 8 rows per lane
@@ -1382,32 +1425,20 @@ ChunkShape chunk_shape(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, 
 // thin, is sliced only when the slices fill nine tenths of their workgroup
 // slots (B=72 H=12: one launch 163.8, 8 slices of 864 chunks 167.6; B=80 in 8
 // of 960: 181.7 / 172.6; B=56 in 7 of 768: 129.2 / 122.8).
-constexpr int64_t kSliceRound = 1024;
-constexpr int64_t kSliceCUs = 256;
-constexpr int64_t kSliceChain = 8;
-constexpr int64_t kSliceMax = 8;
-// Only sequences that run in 512-row chunks (chunk_shape).
+// Only sequences that chunk_shape leaves in 512-row chunks.
 int64_t fwd_slices(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves) {
   const int64_t DG = group_width(v_dtype, D);
   if (B < 2 || DG != D || DG * elem_size(v_dtype) != 128) return 1;
   const int64_t gw = row_groups(v_dtype, D);
-  if (N <= gw * kRSmall * kNWSmall || (!saves && fit_rows(N, gw))) return 1;
+  if (N <= gw * kRSmall * kNWSmall) return 1;
   const int64_t L = chunk_rows(v_dtype, D, ChunkShape{kR, kNW});
   const int64_t chain = (N + L - 1) / L;
   const int64_t per_b = H * chain;  // 512-row chunks of one batch element
-  if (chain > kSliceChain || per_b > kSliceRound || B * per_b <= kSliceRound) return 1;
-  const int64_t b_max = kSliceRound / per_b;
-  const int64_t fewest = (B + b_max - 1) / b_max;
-  if (fewest > kSliceMax) return 1;
-  int64_t best = fewest, best_rounds = 0;
-  for (int64_t n = fewest; n <= fewest + 2 && n <= B && n <= kSliceMax; ++n) {
-    const int64_t rounds = n * (((B + n - 1) / n * per_b + kSliceCUs - 1) / kSliceCUs);
-    if (n == fewest || rounds < best_rounds) best = n, best_rounds = rounds;
-  }
-  const int64_t chunks = (B + best - 1) / best * per_b;
-  const int64_t slots = (chunks + kSliceCUs - 1) / kSliceCUs * kSliceCUs;
-  if (B * per_b >= 4 * kSliceRound && 10 * chunks < 9 * slots) return 1;
-  return best;
+  if (!sliceable(B, chain, per_b, 1)) return 1;
+  if (!saves && fit_rows(B, N, gw, chain, B * per_b, true)) return 1;
+  bool fill;
+  const int64_t n = slice_count(B, per_b, &fill);
+  return B * per_b >= 4 * kSliceRound && !fill ? 1 : n;
 }
 
 // Head dims of the chunked kernels: 16, 32, or any multiple of a full
@@ -1594,31 +1625,61 @@ constexpr int64_t kBwdMidStreams = 48;
 // 24.87 / 31.00; B=3 N=8192 H=16, 768: 27.44 / 33.19).
 constexpr int64_t kBwdMidLo = 192;
 constexpr int64_t kBwdMidHi = 512;
-int bwd_rows_per_lane(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype) {
+// Short sequences: the smallest chunk that holds the whole sequence, of 4 rows x
+// 1 wavefront, 4 x 4, and for 128-byte groups on grids of more than
+// kBwdShortChainGrid streams 8 x 1 and 8 x 4 (chunk_shape has the forward's).
+// Measured (bf16 H=12, projection layout, us, 16-row or 128-row chunks as below /
+// this; a copy of the bytes): D=64 B=1024 N=32 207.4 / 33.2 (29.1), B=512 N=64
+// 109.3 / 32.0 (29.1), B=512 N=100 111.3 / 51.8 (45.5), B=256 N=128 54.4 / 31.7,
+// B=256 N=200 63.3 / 47.1 (45.5), B=192 N=256 60.8 / 44.8 (43.6), B=64 N=100 20.4
+// / 11.9; D=128 B=200 N=100 51.1 / 41.8; D=16 B=400 N=60 97.8 / 22.0, N=200 102.9
+// / 65.8 (narrow groups not beyond 8 rows per group: N=390 143 / 155).  Few
+// streams: 8 x 1 B=8 N=60 9.4 / 10.7; 8 x 4 H=4 B=19 N=193 9.8 / 10.9.
+ChunkShape bwd_shape(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype) {
   const int64_t vw = 16 / elem_size(v_dtype);
   const int64_t DG = bwd_group_width(B, H, N, D, v_dtype);
-  const int64_t L = kNWB * (64 / (DG / vw)) * kRB;
+  const int64_t gw = 64 / (DG / vw);
+  const bool g128 = DG * elem_size(v_dtype) == 128;
+  if (DG * elem_size(v_dtype) <= 128) {
+    if (N <= gw * kRBSmall) return ChunkShape{kRBSmall, 1};
+    const bool many = g128 && B * H * (D / DG) > kBwdShortChainGrid;
+    if (many && N <= gw * kRBMid) return ChunkShape{kRBMid, 1};
+    if (N <= gw * kRBSmall * (g128 ? kNWB : 2)) return ChunkShape{kRBSmall, kNWB};
+    if (many && N <= gw * kRBMid * kNWB) return ChunkShape{kRBMid, kNWB};
+  }
+  const int64_t L = kNWB * gw * kRB;
   const int64_t nstream = B * H * (D / DG);
   const int64_t chain = (N + L - 1) / L;
   const int64_t grid = chain * nstream;
-  const bool g128 = DG * elem_size(v_dtype) == 128;
-  if (g128 && grid > kBwdMidLo && grid <= kBwdMidHi) return kRBMid;
-  if (grid <= kBwdSmallGrid || (grid <= kBwdShortChainGrid && chain <= 4)) return kRBSmall;
-  if (g128 && D / DG >= 2 && grid > kBwdOneRound && nstream >= kBwdMidStreams) return kRBMid;
-  return kRB;
+  if (g128 && grid > kBwdMidLo && grid <= kBwdMidHi) return ChunkShape{kRBMid, kNWB};
+  if (grid <= kBwdSmallGrid || (grid <= kBwdShortChainGrid && chain <= 4)) return ChunkShape{kRBSmall, kNWB};
+  if (g128 && D / DG >= 2 && grid > kBwdOneRound && nstream >= kBwdMidStreams) return ChunkShape{kRBMid, kNWB};
+  return ChunkShape{kRB, kNWB};
 }
 
 int64_t bwd_chunk_rows(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype) {
   const int64_t vw = 16 / elem_size(v_dtype);
   const int64_t lpr = bwd_group_width(B, H, N, D, v_dtype) / vw;
-  return kNWB * (64 / lpr) * bwd_rows_per_lane(B, H, N, D, v_dtype);
+  const ChunkShape c = bwd_shape(B, H, N, D, v_dtype);
+  return c.NW * (64 / lpr) * c.R;
 }
 
 template <typename T, int DG>
-int launch_bwd(const BwdArgs& a, int64_t grid, int R, hipStream_t s) {
+int launch_bwd(const BwdArgs& a, int64_t grid, ChunkShape c, hipStream_t s) {
   constexpr int VW = 16 / (int)sizeof(T);
   constexpr int LPR = DG / VW;
-  if (R == kRB) {
+  const int R = c.R;
+  if (c.NW == 1) {
+    // One chunk of one wavefront per stream (bwd_shape): no look-back.
+    if constexpr (LPR == 8) {
+      auto* const k = R == kRBMid ? scan_bwd<T, LPR, kRBMid, 1, 1, 4> : scan_bwd<T, LPR, kRBSmall, 1, 1, 4>;
+      hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(64), 0, s, a);
+    } else if constexpr (LPR < 8) {
+      hipLaunchKernelGGL((scan_bwd<T, LPR, kRBSmall, 1, 1, 4>), dim3((unsigned)grid), dim3(64), 0, s, a);
+    } else {
+      return fail(KDECAY_ESHAPE, "no one-wavefront backward kernel for %d-channel groups", DG);
+    }
+  } else if (R == kRB) {
     // Batch slices (bwd_slices): one full round each, chains of at most 8.
     if (a.nslice > 1) {
       if constexpr (LPR == 8) {
@@ -1639,7 +1700,7 @@ int launch_bwd(const BwdArgs& a, int64_t grid, int R, hipStream_t s) {
                                                     : one_round;
     hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(kNWB * 64), 0, s, a);
   } else if (R == kRBMid) {
-    // 256-row chunks (bwd_rows_per_lane): one round at four workgroups per CU
+    // 256-row chunks (bwd_shape): one round at four workgroups per CU
     // (window 4, or 8 for chains of more than 8), or several.
     if constexpr (LPR == 8) {
       auto* const w4 = scan_bwd<T, LPR, kRBMid, kNWB, kW, 4>;
@@ -1678,7 +1739,7 @@ int launch_bwd(const BwdArgs& a, int64_t grid, int R, hipStream_t s) {
 }
 
 template <typename T>
-int dispatch_bwd(const BwdArgs& a, int64_t DG, int64_t grid, int R, hipStream_t s) {
+int dispatch_bwd(const BwdArgs& a, int64_t DG, int64_t grid, ChunkShape R, hipStream_t s) {
   switch (DG) {
     case 16: return launch_bwd<T, 16>(a, grid, R, s);
     case 32: return launch_bwd<T, 32>(a, grid, R, s);
@@ -2022,7 +2083,7 @@ int kdecay_scan_fwd_train(const void* V, int v_dtype, const int64_t* v_strides, 
 // (B=32 H=12 in 4: 109.2 / 112.0).  Returns the number of launches.
 int64_t bwd_slices(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype) {
   const int64_t DG = bwd_group_width(B, H, N, D, v_dtype);
-  if (B < 2 || DG != D || DG * elem_size(v_dtype) != 128 || bwd_rows_per_lane(B, H, N, D, v_dtype) != kRB) return 1;
+  if (B < 2 || DG != D || DG * elem_size(v_dtype) != 128 || bwd_shape(B, H, N, D, v_dtype).R != kRB) return 1;
   const int64_t chain = (N + bwd_chunk_rows(B, H, N, D, v_dtype) - 1) / bwd_chunk_rows(B, H, N, D, v_dtype);
   const int64_t grid = B * H * chain;
   if (chain > kSliceChain) return 1;
@@ -2069,7 +2130,7 @@ int kdecay_scan_bwd(const void* V, int v_dtype, const int64_t* v_strides, const 
     if (sizes[k] > 1 && (v_strides[k] % vw || gy_strides[k] % vw || dv_strides[k] % vw))
       return fail(KDECAY_ELAYOUT, "stride %d is not a multiple of 16 bytes", k);
   }
-  const int RB = bwd_rows_per_lane(B, H, N, D, v_dtype);
+  const ChunkShape RB = bwd_shape(B, H, N, D, v_dtype);
   const int64_t Lb = bwd_chunk_rows(B, H, N, D, v_dtype);
   const int64_t nchunk = (N + Lb - 1) / Lb;
   const int64_t DG = bwd_group_width(B, H, N, D, v_dtype);

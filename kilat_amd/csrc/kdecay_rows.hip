@@ -51,6 +51,8 @@ RowSplit row_split(int v_dtype, int64_t D) {
   return s;
 }
 
+int row_slots(const RowSplit& s, int v_dtype) { return s.lpr * (16 / elem_size(v_dtype)); }
+
 struct RowScanArgs {
   ScanArgs s;  // ng: streams per head; flags: [nstream][nchunk][slots] words
   int lpr, gw;  // lanes per row, row groups per wavefront
@@ -237,7 +239,7 @@ void scan_rows(RowScanArgs ra) {
   // Tables, while the rows are in flight.
   for (int k = tid; k <= G; k += NTH) pw[k] = pow_like_torch(lam, (int64_t)k * R);
   for (int r = tid; r < L; r += NTH) {
-    if (row0 + r < a.N) rz[r] = 1.0f / (R == 8 ? z_of_fast(lam, a.t_offset + row0 + r) : z_of(lam, a.t_offset + row0 + r));
+    if (row0 + r < a.N) rz[r] = 1.0f / (R <= 8 ? z_of_fast(lam, a.t_offset + row0 + r) : z_of(lam, a.t_offset + row0 + r));
   }
   float acc[VW];
 #pragma unroll
@@ -482,7 +484,7 @@ void scan_rows_bwd(RowBwdArgs ra) {
   const int ch = vec_channel<VW>(vec0 + ds, D);
   const float lam = a.lam[h];
 
-  // Slots tid (< S <= 128 <= NTH): the state before the chunk's first row (zero
+  // Slots tid (< S <= NTH: at most 128, or 64 with one wavefront): the state before the chunk's first row (zero
   // for the second copy of a channel) and the final-state gradient.  Loaded
   // before the rows and unconditionally (see ChunkBwd::run).
   float cs, cf;
@@ -800,9 +802,10 @@ void scan_rows_bwd(RowBwdArgs ra) {
 }
 
 // Chunk shape: 4 wavefronts of 16 rows per lane; 8 rows for grids that would
-// leave much of the device idle (the limit of kdecay.hip's chunk_shape) and for
-// sequences that an 8-row chunk holds; 8 wavefronts of 8 rows for small grids of
-// long chains (half the hops a carry takes).
+// leave much of the device idle (the limit of kdecay.hip's chunk_shape); 8
+// wavefronts of 8 rows for small grids of long chains (half the hops a carry
+// takes); short sequences take the smallest of 4 rows x 1 wavefront, 8 x 1, 4 x
+// 4 and 8 x 4 that holds them (chunk_shape).
 constexpr int64_t kRowsSmallGrid = 416;
 constexpr int64_t kRowsLongChain = 64;
 
@@ -813,6 +816,10 @@ struct RowShape {
 int64_t rows_chunk(const RowSplit& s, RowShape c) { return (int64_t)c.NW * (64 / s.lpr) * c.R; }
 
 RowShape rows_shape(const RowSplit& s, int64_t B, int64_t H, int64_t N) {
+  const int64_t gw = 64 / s.lpr;
+  if (N <= 4 * gw) return RowShape{4, 1};
+  if (N <= 8 * gw) return RowShape{8, 1};
+  if (N <= 16 * gw) return RowShape{4, 4};
   const int64_t L = rows_chunk(s, RowShape{16, 4}), L8 = L / 2;
   if (N > L8 && (N + L - 1) / L * B * H * s.ng > kRowsSmallGrid) return RowShape{16, 4};
   return RowShape{8, (N + L8 - 1) / L8 >= kRowsLongChain ? 8 : 4};
@@ -826,7 +833,12 @@ int launch_rows_nt(const RowScanArgs& ra, int64_t grid, RowShape c, hipStream_t 
   // The look-back windows as launch_chunked chooses them: wide where few
   // streams make long chains in one round, narrow in several rounds (four
   // workgroups per CU, by registers).
-  if (c.NW == 8) {
+  if (c.NW == 1 || c.R == 4) {  // one chunk per stream
+    auto* const k = c.R == 8    ? scan_rows<TI, TO, 8, 1, 1, 4, false, NT>
+                    : c.NW == 1 ? scan_rows<TI, TO, 4, 1, 1, 4, false, NT>
+                                : scan_rows<TI, TO, 4, 4, 1, 4, false, NT>;
+    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(c.NW * 64), lds, s, ra);
+  } else if (c.NW == 8) {
     hipLaunchKernelGGL((scan_rows<TI, TO, 8, 8, 16, 4, false, NT>), dim3((unsigned)grid), dim3(512), lds, s, ra);
   } else if (c.R == 8) {
     auto* const k = a.nchunk > 16 ? scan_rows<TI, TO, 8, 4, 16, 4, false, NT> : scan_rows<TI, TO, 8, 4, 4, 4, false, NT>;
@@ -872,10 +884,18 @@ constexpr int64_t kRowsBwdSmallGrid = 384;  // chunks of 8 rows per lane
 constexpr int64_t kRowsBwdFullLo = 512;     // chunks of 16
 constexpr int64_t kRowsBwdFullHi = 768;
 
-RowShape rows_bwd_shape(const RowSplit& s, int64_t B, int64_t H, int64_t N) {
+// Short sequences as the forward's, with one wavefront only where its 64 lanes
+// hold a stream's channels (slots), and of 8 rows only for many streams
+// (bwd_shape).
+RowShape rows_bwd_shape(const RowSplit& s, int64_t B, int64_t H, int64_t N, int slots) {
+  const int64_t gw = 64 / s.lpr;
+  if (slots <= 64 && N <= 4 * gw) return RowShape{4, 1};
+  if (slots <= 64 && N <= 8 * gw && B * H * s.ng > kRowsBwdSmallGrid) return RowShape{8, 1};
+  if (N <= 16 * gw) return RowShape{4, 4};
   const int64_t L = rows_chunk(s, RowShape{8, 4}), n = B * H * s.ng;
+  if (N <= L) return RowShape{8, 4};
   const int64_t grid16 = (N + 2 * L - 1) / (2 * L) * n;
-  if (N > L && grid16 > kRowsBwdFullLo && grid16 <= kRowsBwdFullHi) return RowShape{16, 4};
+  if (grid16 > kRowsBwdFullLo && grid16 <= kRowsBwdFullHi) return RowShape{16, 4};
   return RowShape{(N + L - 1) / L * n > kRowsBwdSmallGrid ? 8 : 4, 4};
 }
 
@@ -888,6 +908,11 @@ int launch_rows_bwd_nt(const RowBwdArgs& ra, int64_t grid, RowShape c, hipStream
   const int64_t resident = 4 * (int64_t)cu_count();
   const bool rounds = resident > 0 && grid > resident;
   const int n = a.nchunk;
+  if (c.NW == 1) {  // one chunk of one wavefront per stream
+    auto* const k1 = c.R == 8 ? scan_rows_bwd<T, 8, 1, 1, 4, NT> : scan_rows_bwd<T, 4, 1, 1, 4, NT>;
+    hipLaunchKernelGGL(k1, dim3((unsigned)grid), dim3(64), lds, s, ra);
+    return hip_check("scan_rows_bwd launch");
+  }
   auto* const k = c.R == 16 ? (n > 8 ? scan_rows_bwd<T, 16, 4, 8, 3, NT> : scan_rows_bwd<T, 16, 4, kW, 3, NT>)
                   : c.R == 8 ? (rounds  ? scan_rows_bwd<T, 8, 4, kWRounds, 4, NT>
                                 : n > 8 ? scan_rows_bwd<T, 8, 4, 8, 4, NT>
@@ -919,7 +944,7 @@ size_t kdecay_scan_rows_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t
   const int64_t L = rows_chunk(s, rows_shape(s, B, H, N));
   const int64_t nchunk = (N + L - 1) / L;
   if (nchunk <= 1) return 0;
-  return kHeaderBytes + (size_t)(B * H * s.ng * nchunk * s.lpr * (16 / elem_size(v_dtype))) * sizeof(u64);
+  return kHeaderBytes + (size_t)(B * H * s.ng * nchunk * row_slots(s, v_dtype)) * sizeof(u64);
 }
 
 static int rows_fwd_impl(const void* V, int v_dtype, const int64_t* v_strides, void* out, int out_dtype,
@@ -971,13 +996,16 @@ static int rows_fwd_impl(const void* V, int v_dtype, const int64_t* v_strides, v
   a.hdr = nchunk > 1 ? static_cast<unsigned*>(workspace) : nullptr;
   a.flags = nchunk > 1 ? reinterpret_cast<u64*>(static_cast<char*>(workspace) + kHeaderBytes) : nullptr;
   a.spin_limit = spin_limit();
-  a.state_rows = rows_chunk(sp, rows_bwd_shape(sp, B, H, N));
+  a.state_rows = rows_chunk(sp, rows_bwd_shape(sp, B, H, N, row_slots(sp, v_dtype)));
   a.nsaved = (N + a.state_rows - 1) / a.state_rows;
   a.states = a.nsaved > 1 ? states : nullptr;
   a.rowtab = a.states ? reinterpret_cast<float2*>(states + B * H * D * a.nsaved) : nullptr;
+  // One wavefront's chunks hold sequences that are one backward chunk too: no
+  // states (scan_rows writes the row terms from its other wavefronts).
+  if (shape.NW == 1 && a.states) return fail(KDECAY_EINVAL, "no saving kernel of one wavefront");
   ra.lpr = sp.lpr;
   ra.gw = 64 / sp.lpr;
-  ra.slots = sp.lpr * (16 / elem_size(v_dtype));
+  ra.slots = row_slots(sp, v_dtype);
   ra.f_lpr = make_fastdiv((uint32_t)sp.lpr);
   switch (v_dtype) {
     case KDECAY_F32: return launch_rows<float, float>(ra, grid, shape, s);
@@ -1003,7 +1031,7 @@ size_t kdecay_scan_rows_saved_states_floats(int64_t B, int64_t H, int64_t N, int
   if (B <= 0 || H <= 0 || N <= 0 || !dtype_ok(v_dtype)) return 0;
   const RowSplit sp = row_split(v_dtype, D);
   if (!sp.ok) return 0;
-  const int64_t Lb = rows_chunk(sp, rows_bwd_shape(sp, B, H, N));
+  const int64_t Lb = rows_chunk(sp, rows_bwd_shape(sp, B, H, N, row_slots(sp, v_dtype)));
   const int64_t nsaved = (N + Lb - 1) / Lb;
   return nsaved <= 1 ? 0 : (size_t)(B * H * D * nsaved + 2 * H * N);
 }
@@ -1026,9 +1054,9 @@ size_t kdecay_scan_rows_bwd_workspace_bytes(int64_t B, int64_t H, int64_t N, int
   if (B <= 0 || H <= 0 || N <= 0 || !dtype_ok(v_dtype)) return 0;
   const RowSplit sp = row_split(v_dtype, D);
   if (!sp.ok) return 0;
-  const int64_t Lb = rows_chunk(sp, rows_bwd_shape(sp, B, H, N));
+  const int64_t Lb = rows_chunk(sp, rows_bwd_shape(sp, B, H, N, row_slots(sp, v_dtype)));
   const int64_t nchunk = (N + Lb - 1) / Lb, nstream = B * H * sp.ng;
-  const size_t flags = nchunk > 1 ? (size_t)(nstream * nchunk * sp.lpr * (16 / elem_size(v_dtype))) * sizeof(u64) : 0;
+  const size_t flags = nchunk > 1 ? (size_t)(nstream * nchunk * row_slots(sp, v_dtype)) * sizeof(u64) : 0;
   return kHeaderBytes + flags + (size_t)(nstream * nchunk) * sizeof(u64);
 }
 
@@ -1051,7 +1079,7 @@ int kdecay_scan_rows_bwd(const void* V, int v_dtype, const int64_t* v_strides, c
   const uintptr_t es = (uintptr_t)elem_size(v_dtype);
   if ((uintptr_t)V % es || (uintptr_t)gy % es || (uintptr_t)dV % es)
     return fail(KDECAY_ELAYOUT, "V, gy and dV must be aligned to their elements");
-  const RowShape shape = rows_bwd_shape(sp, B, H, N);
+  const RowShape shape = rows_bwd_shape(sp, B, H, N, row_slots(sp, v_dtype));
   const int64_t Lb = rows_chunk(sp, shape);
   const int64_t nchunk = (N + Lb - 1) / Lb, nstream = B * H * sp.ng, grid = nchunk * nstream;
   if (grid > 0x7fffffffLL) return fail(KDECAY_EINVAL, "problem too large (%lld chunks)", (long long)grid);
@@ -1099,7 +1127,7 @@ int kdecay_scan_rows_bwd(const void* V, int v_dtype, const int64_t* v_strides, c
   a.spin_limit = spin_limit();
   a.per_stream = nstream <= kBwdPerStreamCount;
   a.ndone = bwd_done_count(B, H, sp.ng, nchunk);
-  const int slots = sp.lpr * (16 / (int)es);
+  const int slots = row_slots(sp, v_dtype);
   const size_t flag_bytes = nchunk > 1 ? (size_t)(nstream * nchunk * slots) * sizeof(u64) : 0;
   a.flags = nchunk > 1 ? reinterpret_cast<u64*>(static_cast<char*>(workspace) + kHeaderBytes) : nullptr;
   a.partial = reinterpret_cast<u64*>(static_cast<char*>(workspace) + kHeaderBytes + flag_bytes);

@@ -68,6 +68,30 @@ def _row_vectors_ok(D: int, dtype: torch.dtype) -> bool:
     return left >= 1 and (ng == 1 or left >= 2 or D % vw == 0)
 
 
+
+# Bytes of V from which narrow heads take the row kernels where their rows share
+# memory lines with other heads' (_narrow_rows).
+_NARROW_BYTES = 4 << 20
+
+
+def _narrow_rows(V: torch.Tensor) -> bool:
+    """Whether a head of 16 or 32 channels, less than a 128-byte line, runs on
+    the row kernels although the chunked kernels take it: where a row's line
+    holds other heads' rows too (a projection's view) or the row is 32 bytes.
+    The row kernels number adjacent heads onto one XCD and store pieces of
+    lines through its cache.  Measured (us, chunked / row kernels, forward;
+    backward): bf16 D=16 B=8 H=12 N=4096 projection view 20.1 / 13.6; 28.1 /
+    21.1, contiguous 14.9 / 13.0; 20.0 / 19.9; B=32 H=16 N=1000 view 24.3 / 13.7;
+    39.5 / 41.5, contiguous 20.1 / 12.8; 27.1 / 25.0; bf16 D=32 B=8 H=12 N=4096
+    view 16.6 / 13.1; 32.9 / 24.5, contiguous 13.2 / 13.6 and B=32 H=16 N=1000
+    contiguous 17.5 / 18.9; 26.2 / 29.4; fp32 D=16 B=8 H=12 N=4096 view 16.9 /
+    14.0; 32.2 / 26.0; but B=2 H=6 N=1024 bf16 D=32 view 7.9 / 7.8; 10.3 / 11.6."""
+    D, es = V.shape[3], V.element_size()
+    if D > 32 or D * es >= 128 or V.numel() * es < _NARROW_BYTES:
+        return False
+    return V.stride(2) != D or D * es == 32
+
+
 # One zero-initialised workspace per (device, stream); the kernels keep it
 # consistent from launch to launch, so it is never cleared again.
 _workspaces: dict = {}
@@ -202,6 +226,9 @@ def reserve_workspace(
         tcode = _lib.KDECAY_F32 if code == _lib.KDECAY_F64 else code
         tdtype = torch.float32 if code == _lib.KDECAY_F64 else dtype
         nbytes = max(nbytes, _train_sizes(lib, B, H, N, D, tcode, not chunked_head_dim(D, tdtype))[1])
+    if D <= 32 and _row_vectors_ok(D, dtype):  # narrow heads may take either kernels (_narrow_rows)
+        nbytes = max(nbytes, lib.kdecay_scan_rows_workspace_bytes(B, H, N, D, code),
+                     _train_sizes(lib, B, H, N, D, tcode, True)[1] if backward else 0)
     with _on_device(dev):
         ws = _workspace(dev, _stream_ptr(dev), nbytes)
     return 0 if ws is None else ws.numel()
@@ -286,7 +313,7 @@ class _ScanFn(torch.autograd.Function):
         o_code = _DTYPE_CODE[out_dtype]
         # The saved V also feeds the backward kernel, whose addressing takes
         # a narrower range of row strides than the forward's.
-        rows = not chunked_head_dim(D, V.dtype)
+        ctx.rows = rows = _rows_train(V)
         layout_ok = _row_layout_ok if rows else _train_layout_ok
         Vk = V if layout_ok(V) else V.contiguous()
         out = torch.empty(Vk.shape, dtype=out_dtype, device=dev) if out_dtype != Vk.dtype else torch.empty_like(Vk)
@@ -331,7 +358,7 @@ class _ScanFn(torch.autograd.Function):
         if gy is None:
             gy = torch.zeros_like(Vk)
         gy = gy.to(Vk.dtype)
-        rows = not chunked_head_dim(D, Vk.dtype)
+        rows = ctx.rows
         if not (_row_layout_ok if rows else _train_layout_ok)(gy):
             gy = gy.contiguous()
         dV = torch.empty_like(Vk)
@@ -433,7 +460,8 @@ def global_decay_scan(
                 final.data_ptr() if final is not None else None, B, H, N, D, int(t_offset), stream,
             )
             _lib.check(rc, "kdecay_scan_fwd_sequential")
-        elif chunked_head_dim(D, V.dtype) and _vector_layout_ok(V) and _vector_layout_ok(out):
+        elif (chunked_head_dim(D, V.dtype) and _vector_layout_ok(V) and _vector_layout_ok(out)
+              and not _narrow_rows(V)):
             _chunked(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev)
         elif _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev):
             pass
@@ -512,6 +540,8 @@ def _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, d
 def _rows_train(V: torch.Tensor) -> bool:
     """Whether a training pass over V takes the row kernels (see _rows)."""
     B, H, N, D = V.shape
+    if chunked_head_dim(D, V.dtype) and not _narrow_rows(V):
+        return False
     if not _row_vectors_ok(D, V.dtype):
         return False
     dev = V.device

@@ -258,3 +258,31 @@ def test_rows_backward_infinite_gradient_stays_in_its_channel(hip_device, kdecay
         dv, = torch.autograd.grad(kilat_amd.triton_global_decay(lam, V), V, gy)
         assert torch.isposinf(dv[..., c]).all()
         assert torch.isfinite(dv[..., :c]).all() and torch.isfinite(dv[..., c + 1:]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname,D", [("bf16", 16), ("bf16", 32), ("f16", 32), ("f32", 16)])
+def test_narrow_heads_on_the_row_kernels(hip_device, kdecay_lib, dname, D, monkeypatch):
+    """Heads of 16 and 32 channels from the projection layout, large enough for
+    the row kernels, against the chunked kernels the same call takes when it is
+    not: forward with a carried state, and the gradients."""
+    from kilat_amd import triton_ops
+
+    dtype = DTYPES[dname]
+    B, H, N = 6, 12, 2100
+    B *= 64 // (D * torch.empty((), dtype=dtype).element_size())
+    lam = lam_uniform(H, 0.5, 0.999, torch.Generator().manual_seed(9)).to(hip_device).requires_grad_()
+    V = torch.randn(B, N, H, D, device=hip_device).to(dtype).transpose(1, 2).requires_grad_()
+    gy = torch.randn(B, N, H, D, device=hip_device).to(dtype).transpose(1, 2)
+    init = torch.randn(B, H, D, device=hip_device)
+    assert triton_ops._narrow_rows(V) and not triton_ops._narrow_rows(V[:1, :, :100])
+    got = []
+    for _ in range(2):
+        with torch.no_grad():
+            y, fin = kilat_amd.global_decay_scan(lam, V, initial_state=init, return_final_state=True, t_offset=3)
+        dv, dl = torch.autograd.grad(kilat_amd.triton_global_decay(lam, V), (V, lam), gy)
+        got.append((y, fin, dv, dl))
+        monkeypatch.setattr(triton_ops, "_NARROW_BYTES", 1 << 60)
+    (y, fin, dv, dl), (y0, fin0, dv0, dl0) = got
+    assert rel_err(y, y0) <= TOL[dtype] and rel_err(fin, fin0) <= 1e-5 and rel_err(dv, dv0) <= TOL[dtype]
+    assert float((dl - dl0).abs().max() / dl0.abs().max()) <= 1e-4

@@ -1,4 +1,5 @@
-"""Build recipe of ``libkdecay.so``: one hipcc compilation per source for gfx950, then a link.
+"""Build recipe: ``libkdecay.so`` (one hipcc compilation per source for gfx950, then a link) and
+``_native.so``, the host path of the Python functions (g++ against torch's headers).
 
 Run ``python -m kilat_amd._build`` (or ``__graft_entry__.build()``).  The
 library is written in-tree next to this file, where ``kilat_amd._lib`` loads it.
@@ -16,6 +17,8 @@ ROOT = os.path.dirname(HERE)
 SOURCES = [os.path.join(HERE, "csrc", name) for name in ("kdecay.hip", "kdecay_rows.hip")]
 INCLUDE = os.path.join(ROOT, "include")
 LIBRARY = os.path.join(HERE, "libkdecay.so")
+NATIVE_SOURCE = os.path.join(HERE, "csrc", "native.cpp")
+NATIVE = os.path.join(HERE, "_native.so")
 
 # -packed-fp32-ops: no v_pk_*_f32 in the device code.
 # -mcode-object-version=5: loadable by torch's bundled ROCm 7.0 runtime.
@@ -67,5 +70,38 @@ def build_library(verbose: bool = False) -> str:
     return LIBRARY
 
 
+def build_native(verbose: bool = False) -> str:
+    """Compile csrc/native.cpp into _native.so (after libkdecay.so, which it links); returns its path."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    tmp = NATIVE + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE]
+    for path in [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]:
+        cmd += ["-isystem", path]
+    cmd += [NATIVE_SOURCE, "-o", tmp, "-L", HERE, "-lkdecay", "-Wl,-rpath,$ORIGIN"]
+    for path in cpp_extension.library_paths():
+        cmd += ["-L", path]
+    cmd += ["-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError("g++ failed:\n" + proc.stdout)
+    if verbose and proc.stdout.strip():
+        print(proc.stdout, flush=True)
+    os.replace(tmp, NATIVE)
+    return NATIVE
+
+
+def build(verbose: bool = False) -> None:
+    build_library(verbose)
+    build_native(verbose)
+
+
 if __name__ == "__main__":
-    print(build_library(verbose="-v" in sys.argv))
+    build(verbose="-v" in sys.argv)
+    print(LIBRARY, NATIVE)

@@ -24,6 +24,23 @@ import torch
 
 from . import _lib
 
+try:
+    from . import _native  # the host path in C++ (csrc/native.cpp)
+except ImportError as e:
+    class _Missing:
+        """Stands in for _native until it is built: any use raises."""
+
+        def __init__(self, why: str) -> None:
+            self.why = why
+
+        def __getattr__(self, name: str):
+            raise RuntimeError(
+                f"kilat_amd: _native.so cannot be loaded ({self.why}); build it with `python -m kilat_amd._build` "
+                "(there is no fallback)"
+            )
+
+    _native = _Missing(str(e))
+
 _DTYPE_CODE = {
     torch.float32: _lib.KDECAY_F32,
     torch.bfloat16: _lib.KDECAY_BF16,
@@ -55,45 +72,13 @@ def _padded_head_dim(D: int, dtype: torch.dtype) -> int:
 
 
 def _row_vectors_ok(D: int, dtype: torch.dtype) -> bool:
-    """Head dims kdecay_scan_fwd_rows splits into 16-byte vectors (row_split in
-    kdecay_rows.hip): whole rows of up to 16 vectors, wider ones in the fewest
-    equal streams; not less than one vector, and not a last stream of one
-    vector that overlaps the stream before it."""
-    vw = _GROUP[dtype] // 8
-    if D < vw:
-        return False
-    nv = -(-D // vw)
-    ng = -(-nv // 16)
-    left = nv - (ng - 1) * -(-nv // ng)
-    return left >= 1 and (ng == 1 or left >= 2 or D % vw == 0)
-
-
-
-# Bytes of V from which narrow heads take the row kernels where their rows share
-# memory lines with other heads' (_narrow_rows).
-_NARROW_BYTES = 4 << 20
-
-
-def _narrow_rows(V: torch.Tensor) -> bool:
-    """Whether a head of 16 or 32 channels, less than a 128-byte line, runs on
-    the row kernels although the chunked kernels take it: where a row's line
-    holds other heads' rows too (a projection's view) or the row is 32 bytes.
-    The row kernels number adjacent heads onto one XCD and store pieces of
-    lines through its cache.  Measured (us, chunked / row kernels, forward;
-    backward): bf16 D=16 B=8 H=12 N=4096 projection view 20.1 / 13.6; 28.1 /
-    21.1, contiguous 14.9 / 13.0; 20.0 / 19.9; B=32 H=16 N=1000 view 24.3 / 13.7;
-    39.5 / 41.5, contiguous 20.1 / 12.8; 27.1 / 25.0; bf16 D=32 B=8 H=12 N=4096
-    view 16.6 / 13.1; 32.9 / 24.5, contiguous 13.2 / 13.6 and B=32 H=16 N=1000
-    contiguous 17.5 / 18.9; 26.2 / 29.4; fp32 D=16 B=8 H=12 N=4096 view 16.9 /
-    14.0; 32.2 / 26.0; but B=2 H=6 N=1024 bf16 D=32 view 7.9 / 7.8; 10.3 / 11.6."""
-    D, es = V.shape[3], V.element_size()
-    if D > 32 or D * es >= 128 or V.numel() * es < _NARROW_BYTES:
-        return False
-    return V.stride(2) != D or D * es == 32
+    """Head dims kdecay_scan_fwd_rows splits into 16-byte vectors."""
+    return _native.row_vectors_ok(D, 128 // _GROUP[dtype])
 
 
 # One zero-initialised workspace per (device, stream); the kernels keep it
-# consistent from launch to launch, so it is never cleared again.
+# consistent from launch to launch, so it is never cleared again.  _native looks
+# them up here on every call.
 _workspaces: dict = {}
 # Workspaces replaced by a larger one.  A HIP graph captured with a workspace
 # keeps its raw address, so a workspace that was ever handed to a launch is
@@ -118,34 +103,13 @@ def _dtype_code(t: torch.Tensor, name: str) -> int:
         raise TypeError(f"kilat_amd: {name} dtype {t.dtype} is not float32/bfloat16/float16/float64") from None
 
 
+# Layouts the kernels take (see native.cpp).
 def _vector_layout_ok(t: torch.Tensor) -> bool:
-    """The chunked kernel's layout rule: d-stride 1, 16-byte base, and every
-    other stride a multiple of 16 bytes (size-1 dims excepted).  Called only
-    for head dims the chunked kernels take, whose rows are whole 16-byte
-    vectors."""
-    if t.data_ptr() & 15:
-        return False
-    vw = 16 // t.element_size()
-    sz, st = t.shape, t.stride()
-    return ((st[3] == 1 or sz[3] == 1) and (st[2] % vw == 0 or sz[2] == 1) and (st[1] % vw == 0 or sz[1] == 1)
-            and (st[0] % vw == 0 or sz[0] == 1))
+    return _native.vector_layout_ok(t)
 
 
 def _bwd_rows_fit(t: torch.Tensor) -> bool:
-    """The backward kernel's addressing rule: it reads one chunk of rows of V
-    and of the upstream gradient through 32-bit byte offsets, so a chunk's
-    rows must span less than 2^31 bytes (the library rejects other row
-    strides).  A chunk holds at most 4 wavefronts x (64 lanes / lanes per
-    row) x 16 rows per lane; the bound below uses that largest chunk, so a
-    tensor that passes is accepted whatever chunk size the library picks
-    (whole 256-byte rows, 16 lanes each, make 256-row chunks: fewer rows)."""
-    B, H, N, D = t.shape
-    es = t.element_size()
-    lanes_per_row = min(D, 128 // es) * es // 16
-    if N <= 1 or lanes_per_row < 1:
-        return True
-    max_rows = 4 * (64 // lanes_per_row) * 16
-    return max_rows * t.stride(2) * es <= 0x7FFFFFFF
+    return _native.bwd_rows_fit(t.shape[2], t.shape[3], t.element_size(), t.stride(2))
 
 
 if hasattr(torch._C, "_cuda_getCurrentRawStream"):
@@ -226,7 +190,7 @@ def reserve_workspace(
         tcode = _lib.KDECAY_F32 if code == _lib.KDECAY_F64 else code
         tdtype = torch.float32 if code == _lib.KDECAY_F64 else dtype
         nbytes = max(nbytes, _train_sizes(lib, B, H, N, D, tcode, not chunked_head_dim(D, tdtype))[1])
-    if D <= 32 and _row_vectors_ok(D, dtype):  # narrow heads may take either kernels (_narrow_rows)
+    if D <= 32 and _row_vectors_ok(D, dtype):  # narrow heads may take either kernels (narrow_rows in native.cpp)
         nbytes = max(nbytes, lib.kdecay_scan_rows_workspace_bytes(B, H, N, D, code),
                      _train_sizes(lib, B, H, N, D, tcode, True)[1] if backward else 0)
     with _on_device(dev):
@@ -264,15 +228,6 @@ def _lam32(lam: torch.Tensor, H: int, device: torch.device) -> torch.Tensor:
     return lam.detach().reshape(H).to(device=device, dtype=torch.float32).contiguous()
 
 
-def _train_layout_ok(t: torch.Tensor) -> bool:
-    return _vector_layout_ok(t) and _bwd_rows_fit(t)
-
-
-def _row_layout_ok(t: torch.Tensor) -> bool:
-    """The row kernels' layout rule: d-stride 1."""
-    return t.stride(3) == 1
-
-
 def _train_sizes(lib, B: int, H: int, N: int, D: int, v_code: int, rows: bool) -> Tuple[int, int]:
     """Floats of the saved states, and bytes of workspace that the training
     forward and its backward need."""
@@ -290,101 +245,6 @@ def _workspace_short_in_capture(dev: torch.device, stream: int, nbytes: int) -> 
     nbytes (it cannot grow there)."""
     ws = _workspaces.get((dev.index, stream))
     return (nbytes if ws is None else nbytes - ws.numel()) > 0 and torch.cuda.is_current_stream_capturing()
-
-
-class _ScanFn(torch.autograd.Function):
-    """The chunked scan with a backward (kdecay_scan_fwd_train / kdecay_scan_bwd).
-
-    Inputs: lam (fp32 [H], differentiable), V, init (fp32 [B,H,D] or None),
-    t_offset, out dtype, sequential.  Outputs: (y, final state).  The
-    reference's GPU path has no backward; its CPU path is differentiated by
-    torch autograd through triton_ops.py:240-246, which this replaces on HIP
-    tensors.  With sequential=True, y and the final state are then rewritten
-    by the sequential kernel (its bits), while the backward uses the states
-    the chunked training forward saved (equal to tolerance).  Head dims the
-    chunked kernels do not take run on the row kernels (_train_sizes).
-    """
-
-    @staticmethod
-    def forward(ctx, lam32, V, init32, t_offset, out_dtype, sequential=False):
-        B, H, N, D = V.shape
-        dev = V.device
-        v_code = _DTYPE_CODE[V.dtype]
-        o_code = _DTYPE_CODE[out_dtype]
-        # The saved V also feeds the backward kernel, whose addressing takes
-        # a narrower range of row strides than the forward's.
-        ctx.rows = rows = _rows_train(V)
-        layout_ok = _row_layout_ok if rows else _train_layout_ok
-        Vk = V if layout_ok(V) else V.contiguous()
-        out = torch.empty(Vk.shape, dtype=out_dtype, device=dev) if out_dtype != Vk.dtype else torch.empty_like(Vk)
-        if not (_row_layout_ok if rows else _vector_layout_ok)(out):
-            out = torch.empty(Vk.shape, dtype=out_dtype, device=dev)
-        final = torch.empty((B, H, D), dtype=torch.float32, device=dev)
-        lib = _lib.load()
-        nst, nbytes = _train_sizes(lib, B, H, N, D, v_code, rows)
-        states = torch.empty(max(nst, 1), dtype=torch.float32, device=dev)
-        fwd_train = lib.kdecay_scan_fwd_rows_train if rows else lib.kdecay_scan_fwd_train
-        with _on_device(dev):
-            stream = _stream_ptr(dev)
-            ws = _workspace(dev, stream, nbytes)
-            rc = fwd_train(
-                Vk.data_ptr(), v_code, _lib.strides4(Vk.stride()),
-                out.data_ptr(), o_code, _lib.strides4(out.stride()),
-                lam32.data_ptr(), init32.data_ptr() if init32 is not None else None, final.data_ptr(),
-                states.data_ptr(), states.numel(), B, H, N, D, int(t_offset),
-                ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, stream,
-            )
-        _lib.check(rc, "kdecay_scan_fwd_train")
-        if sequential:
-            with _on_device(dev):
-                rc = lib.kdecay_scan_fwd_sequential(
-                    Vk.data_ptr(), v_code, _lib.strides4(Vk.stride()),
-                    out.data_ptr(), o_code, _lib.strides4(out.stride()),
-                    lam32.data_ptr(), init32.data_ptr() if init32 is not None else None, final.data_ptr(),
-                    B, H, N, D, int(t_offset), _stream_ptr(dev),
-                )
-            _lib.check(rc, "kdecay_scan_fwd_sequential")
-        ctx.t_offset = int(t_offset)
-        ctx.has_init = init32 is not None
-        ctx.save_for_backward(lam32, Vk, init32 if init32 is not None else final.new_empty(0), states)
-        return out, final
-
-    @staticmethod
-    def backward(ctx, gy, gfin):
-        lam32, Vk, init32, states = ctx.saved_tensors
-        B, H, N, D = Vk.shape
-        dev = Vk.device
-        v_code = _DTYPE_CODE[Vk.dtype]
-        if gy is None:
-            gy = torch.zeros_like(Vk)
-        gy = gy.to(Vk.dtype)
-        rows = ctx.rows
-        if not (_row_layout_ok if rows else _train_layout_ok)(gy):
-            gy = gy.contiguous()
-        dV = torch.empty_like(Vk)
-        if not (_row_layout_ok if rows else _vector_layout_ok)(dV):
-            dV = torch.empty(Vk.shape, dtype=Vk.dtype, device=dev)
-        dlam = torch.empty(H, dtype=torch.float32, device=dev)
-        dinit = torch.empty((B, H, D), dtype=torch.float32, device=dev) if ctx.has_init else None
-        g_fin = gfin.to(torch.float32).contiguous() if gfin is not None else None
-        lib = _lib.load()
-        with _on_device(dev):
-            stream = _stream_ptr(dev)
-            nbytes = (lib.kdecay_scan_rows_bwd_workspace_bytes if rows else lib.kdecay_scan_bwd_workspace_bytes)(
-                B, H, N, D, v_code)
-            ws = _workspace(dev, stream, nbytes)
-            rc = (lib.kdecay_scan_rows_bwd if rows else lib.kdecay_scan_bwd)(
-                Vk.data_ptr(), v_code, _lib.strides4(Vk.stride()),
-                gy.data_ptr(), _lib.strides4(gy.stride()),
-                dV.data_ptr(), _lib.strides4(dV.stride()),
-                lam32.data_ptr(), init32.data_ptr() if ctx.has_init else None, states.data_ptr(),
-                g_fin.data_ptr() if g_fin is not None else None,
-                dlam.data_ptr(), dinit.data_ptr() if dinit is not None else None,
-                B, H, N, D, ctx.t_offset,
-                ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, stream,
-            )
-        _lib.check(rc, "kdecay_scan_bwd")
-        return dlam, dV, dinit, None, None, None
 
 
 def _needs_grad(*ts) -> bool:
@@ -421,6 +281,16 @@ def global_decay_scan(
     dtype first.  A float64 V takes float64 out only; with a gradient it runs
     the fp32 training kernels on V rounded to fp32.
     """
+    if out is None and algorithm == "chunked":
+        r = _native.scan(lam, V, initial_state, bool(return_final_state), t_offset, out_dtype)
+        if r is not None:
+            return r
+    return _scan(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, algorithm)
+
+
+def _scan(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, algorithm):
+    """global_decay_scan for any arguments: checks, conversions, copies and
+    padding around the kernels (_native.scan takes the calls that need none)."""
     _require_hip(V, "V")
     if V.dim() != 4:
         raise ValueError(f"kilat_amd: V must be [B,H,N,D], got shape {tuple(V.shape)}")
@@ -461,7 +331,7 @@ def global_decay_scan(
             )
             _lib.check(rc, "kdecay_scan_fwd_sequential")
         elif (chunked_head_dim(D, V.dtype) and _vector_layout_ok(V) and _vector_layout_ok(out)
-              and not _narrow_rows(V)):
+              and not _native.narrow_rows(V)):
             _chunked(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev)
         elif _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev):
             pass
@@ -540,7 +410,7 @@ def _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, d
 def _rows_train(V: torch.Tensor) -> bool:
     """Whether a training pass over V takes the row kernels (see _rows)."""
     B, H, N, D = V.shape
-    if chunked_head_dim(D, V.dtype) and not _narrow_rows(V):
+    if chunked_head_dim(D, V.dtype) and not _native.narrow_rows(V):
         return False
     if not _row_vectors_ok(D, V.dtype):
         return False
@@ -552,7 +422,7 @@ def _rows_train(V: torch.Tensor) -> bool:
 
 def _scan_with_grad(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, algorithm):
     """global_decay_scan when a gradient is required: the chunked training
-    forward and backward under _ScanFn (the row kernels for head dims the
+    forward and backward (scan_train in native.cpp; the row kernels for head dims the
     chunked ones do not take), with differentiable zero-padding of the channels
     for head dims neither takes, and a differentiable copy into `out` when one
     is given."""
@@ -606,7 +476,7 @@ def _scan_with_grad(lam, V, initial_state, return_final_state, t_offset, out, ou
     o_dtype = out_dtype or V.dtype
     if o_dtype not in (V.dtype, torch.float32):
         raise TypeError("kilat_amd: out dtype must be V's dtype or float32")
-    y, final = _ScanFn.apply(lam32, V, init32, int(t_offset), o_dtype, algorithm == "sequential")
+    y, final = _native.scan_train(lam32, V, init32, int(t_offset), o_dtype, _rows_train(V), algorithm == "sequential")
     if return_final_state:
         return y, final
     return y
@@ -623,7 +493,8 @@ def triton_global_decay(lam_scores: torch.Tensor, V: torch.Tensor) -> torch.Tens
     carries a backward (dV and dlam on the GPU), as the reference's CPU path
     does through torch autograd; its GPU path has none.
     """
-    return global_decay_scan(lam_scores, V)
+    y = _native.scan(lam_scores, V, None, False, 0, None)
+    return _scan(lam_scores, V, None, False, 0, None, None, "chunked") if y is None else y
 
 
 def decay_step(
@@ -648,6 +519,9 @@ def decay_step(
     tensor [B] of per-sequence positions.  new_state may be past_state itself
     (in-place).  Returns (out [B,H,D] out_dtype, new_state [B,H,D] fp32).
     """
+    r = _native.decay_step(lam, past_state, v_t, t_pos, out, new_state, out_dtype)
+    if r is not None:
+        return r
     _require_hip(past_state, "past_state")
     if past_state.dim() != 3:
         raise ValueError(f"kilat_amd: past_state must be [B,H,D], got {tuple(past_state.shape)}")

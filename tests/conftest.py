@@ -14,11 +14,13 @@ def pytest_configure(config):
 
 @pytest.fixture(scope="session")
 def kdecay_lib():
-    """libkdecay.so, built in-tree if it is not there yet."""
+    """libkdecay.so (and the host path that links it), built in-tree if not there yet."""
     from kilat_amd import _build, _lib
 
     if not os.path.exists(_build.LIBRARY):
         _build.build_library()
+    if not os.path.exists(_build.NATIVE):
+        _build.build_native()
     return _lib.load()
 
 

@@ -262,27 +262,31 @@ def test_rows_backward_infinite_gradient_stays_in_its_channel(hip_device, kdecay
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("dname,D", [("bf16", 16), ("bf16", 32), ("f16", 32), ("f32", 16)])
-def test_narrow_heads_on_the_row_kernels(hip_device, kdecay_lib, dname, D, monkeypatch):
+def test_narrow_heads_on_the_row_kernels(hip_device, kdecay_lib, dname, D):
     """Heads of 16 and 32 channels from the projection layout, large enough for
-    the row kernels, against the chunked kernels the same call takes when it is
-    not: forward with a carried state, and the gradients."""
-    from kilat_amd import triton_ops
+    the row kernels, against the chunked kernels that smaller batches of the same
+    rows take: forward with a carried state, and the gradients."""
+    from kilat_amd import _native
 
     dtype = DTYPES[dname]
     B, H, N = 6, 12, 2100
     B *= 64 // (D * torch.empty((), dtype=dtype).element_size())
     lam = lam_uniform(H, 0.5, 0.999, torch.Generator().manual_seed(9)).to(hip_device).requires_grad_()
-    V = torch.randn(B, N, H, D, device=hip_device).to(dtype).transpose(1, 2).requires_grad_()
+    V = torch.randn(B, N, H, D, device=hip_device).to(dtype).transpose(1, 2)
     gy = torch.randn(B, N, H, D, device=hip_device).to(dtype).transpose(1, 2)
     init = torch.randn(B, H, D, device=hip_device)
-    assert triton_ops._narrow_rows(V) and not triton_ops._narrow_rows(V[:1, :, :100])
-    got = []
-    for _ in range(2):
+
+    def call(rows):
+        v = V[rows].requires_grad_()
         with torch.no_grad():
-            y, fin = kilat_amd.global_decay_scan(lam, V, initial_state=init, return_final_state=True, t_offset=3)
-        dv, dl = torch.autograd.grad(kilat_amd.triton_global_decay(lam, V), (V, lam), gy)
-        got.append((y, fin, dv, dl))
-        monkeypatch.setattr(triton_ops, "_NARROW_BYTES", 1 << 60)
-    (y, fin, dv, dl), (y0, fin0, dv0, dl0) = got
+            y, fin = kilat_amd.global_decay_scan(lam, v, initial_state=init[rows], return_final_state=True, t_offset=3)
+        dv, dl = torch.autograd.grad(kilat_amd.triton_global_decay(lam, v), (v, lam), gy[rows])
+        return y, fin, dv, dl
+
+    assert _native.narrow_rows(V) and not _native.narrow_rows(V[:1])
+    y, fin, dv, dl = call(slice(None))
+    parts = [call(slice(b, b + 1)) for b in range(B)]
+    y0, fin0, dv0 = (torch.cat([p[k] for p in parts]) for k in range(3))
+    dl0 = sum(p[3].double() for p in parts)
     assert rel_err(y, y0) <= TOL[dtype] and rel_err(fin, fin0) <= 1e-5 and rel_err(dv, dv0) <= TOL[dtype]
     assert float((dl - dl0).abs().max() / dl0.abs().max()) <= 1e-4

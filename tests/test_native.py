@@ -1,0 +1,94 @@
+"""The host path in C++ (_native): it takes the calls whose arguments the kernels
+read as they are, with the general path's results, and leaves the others to it."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+import kilat_amd
+from kilat_amd import triton_ops
+from tests.decay_cases import lam_uniform
+
+DTYPES = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16, "f64": torch.float64}
+
+
+@pytest.mark.parametrize("dname", ["f32", "bf16", "f64"])
+def test_head_dims_agree(kdecay_lib, dname):
+    from kilat_amd import _native
+
+    es = torch.empty((), dtype=DTYPES[dname]).element_size()
+    for D in range(1, 700):
+        assert _native.chunked_head_dim(D, es) == kilat_amd.chunked_head_dim(D, DTYPES[dname]), D
+
+
+def test_cpu_and_foreign_arguments_are_left(kdecay_lib):
+    from kilat_amd import _native
+
+    lam, V = torch.rand(3), torch.randn(2, 3, 5, 64)
+    assert _native.scan(lam, V, None, False, 0, None) is None
+    assert _native.scan(lam, [1], None, False, 0, None) is None
+    assert _native.scan(None, V, None, False, 0.0, None) is None
+    assert _native.decay_step(lam, V[:, :, 0], V[:, :, 0], 3, None, None, torch.float32) is None
+    with pytest.raises(RuntimeError, match="cpu"):
+        kilat_amd.triton_global_decay(lam, V)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname,out,D", [("bf16", None, 64), ("bf16", "f32", 64), ("f16", None, 80), ("f32", None, 32),
+                                         ("f32", None, 50), ("f64", None, 48), ("bf16", None, 16)])
+def test_scan_equals_the_general_path(hip_device, kdecay_lib, dname, out, D):
+    from kilat_amd import _native
+
+    dtype, out = DTYPES[dname], DTYPES[out] if out else None
+    g = torch.Generator().manual_seed(1400 + D)
+    lam = lam_uniform(3, 0.5, 0.9999, g).to(hip_device)
+    for N in (7, 700):
+        for V in (torch.randn(2, 3, N, D, device=hip_device).to(dtype),
+                  torch.randn(2, N, 3, D, device=hip_device).to(dtype).transpose(1, 2),
+                  torch.randn(2, 3, 2 * N, D, device=hip_device).to(dtype)[:, :, ::2],
+                  torch.randn(1, 3, N, D, device=hip_device).to(dtype).expand(2, 3, N, D)):
+            for init in (None, torch.randn(2, 3, D, device=hip_device)):
+                slow = triton_ops._scan(lam, V, init, True, 5, None, out, "chunked")  # also grows the workspace
+                fast = _native.scan(lam, V, init, True, 5, out)
+                assert fast is not None and all(torch.equal(a, b) for a, b in zip(fast, slow))
+                assert fast[0].stride() == slow[0].stride() and fast[0].dtype == slow[0].dtype
+
+
+@pytest.mark.gpu
+def test_calls_left_to_the_general_path(hip_device, kdecay_lib):
+    """Arguments that need a conversion, a copy, padding or an error."""
+    from kilat_amd import _native
+
+    lam = torch.rand(3, device=hip_device)
+    V = torch.randn(2, 3, 40, 64, device=hip_device)
+    init = torch.randn(2, 3, 64, device=hip_device)
+    for args in ((lam.double(), V, None, False, 0, None), (lam[:2], V, None, False, 0, None),
+                 (lam.cpu(), V, None, False, 0, None), (lam, V.int(), None, False, 0, None),
+                 (lam, V[0], None, False, 0, None), (lam, V[:, :, :0], None, False, 0, None),
+                 (lam, V[..., :3].contiguous(), None, False, 0, None), (lam, V[..., ::2], None, False, 0, None),
+                 (lam, V, init.half(), False, 0, None), (lam, V, init[..., :3], False, 0, None),
+                 (lam, V, None, False, 0, torch.float16), (lam, V.double().requires_grad_(), None, False, 0, None)):
+        assert _native.scan(*args) is None
+    s, v = init, init.half()
+    for args in ((lam, s.half(), v, 3, None, None, torch.float32), (lam, s, v.double(), 3, None, None, torch.float32),
+                 (lam, s, v.transpose(0, 1), 3, None, None, torch.float32), (lam, s, v, 3.0, None, None, torch.float32),
+                 (lam, s, v, torch.tensor([1, 2]), None, None, torch.float32),
+                 (lam, s, v, 3, None, s[:1], torch.float32), (lam, s, v, 3, None, None, torch.float64)):
+        assert _native.decay_step(*args) is None
+
+
+@pytest.mark.gpu
+def test_step_equals_the_general_path(hip_device, kdecay_lib):
+    lam = lam_uniform(3, 0.5, 0.9999, torch.Generator().manual_seed(3)).to(hip_device)
+    s = torch.randn(2, 3, 40, device=hip_device)
+    pos = torch.tensor([4, 900], dtype=torch.int32, device=hip_device)
+    for vt in (torch.float32, torch.bfloat16, torch.float16):
+        v = torch.randn(2, 1, 120, device=hip_device).to(vt)
+        for t_pos, same in ((9, torch.tensor([9, 9])), (pos, pos.cpu())):
+            for ot in (torch.float32, torch.bfloat16):
+                o, n = kilat_amd.decay_step(lam, s, v, t_pos, out_dtype=ot)
+                o2, n2 = kilat_amd.decay_step(lam, s, v, same, out_dtype=ot)  # a host int64 vector: the general path
+                assert torch.equal(o, o2) and torch.equal(n, n2) and o.dtype == ot
+        out, state = torch.empty_like(o, dtype=torch.float32), s.clone()
+        r = kilat_amd.decay_step(lam, state, v, pos, out=out, new_state=state)
+        assert r[0] is out and r[1] is state and torch.equal(state, n)

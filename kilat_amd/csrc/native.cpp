@@ -105,8 +105,10 @@ hipStream_t stream_of(const at::Device& d) { return c10::hip::getCurrentHIPStrea
 // dictionary is the one place that holds workspaces; nothing here keeps one from
 // call to call.  Called with the GIL held.
 Tensor find_workspace(const at::Device& d, hipStream_t stream) {
-  static PyObject* const all =
-      py::module_::import("kilat_amd.triton_ops").attr("_workspaces").cast<py::dict>().release().ptr();
+  // Set under the GIL without a static's guard: the import may give the GIL up,
+  // and a thread waiting for the guard would keep it from coming back.
+  static PyObject* all = nullptr;
+  if (!all) all = py::module_::import("kilat_amd.triton_ops").attr("_workspaces").cast<py::dict>().release().ptr();
   const py::tuple key = py::make_tuple(static_cast<int>(d.index()), reinterpret_cast<uintptr_t>(stream));
   PyObject* const t = PyDict_GetItemWithError(all, key.ptr());
   if (!t) {

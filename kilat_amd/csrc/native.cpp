@@ -264,8 +264,9 @@ py::object scan(const py::object& lam_o, const py::object& V_o, const py::object
   const int v_code = dtype_code(vt), o_code = dtype_code(ot);
   if (v_code < 0 || (ot != vt && (ot != at::kFloat || vt == at::kDouble))) return py::none();
   if (!plain_lam(lam, H, d) || (init.defined() && !plain_state(init, B, H, D, d))) return py::none();
-  const int64_t t_offset = PyLong_AsLongLong(t_offset_o.ptr());
-  if (t_offset == -1 && PyErr_Occurred()) throw py::error_already_set();
+  int overflow = 0;  // the general path takes integers beyond 64 bits as ctypes does
+  const int64_t t_offset = PyLong_AsLongLongAndOverflow(t_offset_o.ptr(), &overflow);
+  if (overflow) return py::none();
 
   const bool narrow = narrow_rows(V), chunked = chunked_head_dim(D, V.element_size()) && !narrow;
   if (!chunked && !row_vectors_ok(D, V.element_size())) return py::none();
@@ -331,8 +332,9 @@ py::object decay_step(const py::object& lam_o, const py::object& state_o, const 
   const int32_t* pos = nullptr;
   int64_t pos_all = 0;
   if (PyLong_CheckExact(pos_o.ptr())) {
-    pos_all = PyLong_AsLongLong(pos_o.ptr());
-    if (pos_all == -1 && PyErr_Occurred()) throw py::error_already_set();
+    int overflow = 0;
+    pos_all = PyLong_AsLongLongAndOverflow(pos_o.ptr(), &overflow);
+    if (overflow) return py::none();
   } else {
     if (!plain_tensor(pos_o.ptr())) return py::none();
     const Tensor& p = THPVariable_Unpack(pos_o.ptr());

@@ -66,12 +66,13 @@ def test_calls_left_to_the_general_path(hip_device, kdecay_lib):
                  (lam.cpu(), V, None, False, 0, None), (lam, V.int(), None, False, 0, None),
                  (lam, V[0], None, False, 0, None), (lam, V[:, :, :0], None, False, 0, None),
                  (lam, V[..., :3].contiguous(), None, False, 0, None), (lam, V[..., ::2], None, False, 0, None),
-                 (lam, V, init.half(), False, 0, None), (lam, V, init[..., :3], False, 0, None),
+                 (lam, V, None, False, 2**64, None), (lam, V, init.half(), False, 0, None), (lam, V, init[..., :3], False, 0, None),
                  (lam, V, None, False, 0, torch.float16), (lam, V.double().requires_grad_(), None, False, 0, None)):
         assert _native.scan(*args) is None
     s, v = init, init.half()
     for args in ((lam, s.half(), v, 3, None, None, torch.float32), (lam, s, v.double(), 3, None, None, torch.float32),
                  (lam, s, v.transpose(0, 1), 3, None, None, torch.float32), (lam, s, v, 3.0, None, None, torch.float32),
+                 (lam, s, v, 2**64, None, None, torch.float32),
                  (lam, s, v, torch.tensor([1, 2]), None, None, torch.float32),
                  (lam, s, v, 3, None, s[:1], torch.float32), (lam, s, v, 3, None, None, torch.float64)):
         assert _native.decay_step(*args) is None

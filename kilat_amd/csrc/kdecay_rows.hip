@@ -883,6 +883,18 @@ int launch_rows(const RowScanArgs& ra, int64_t grid, RowShape c, hipStream_t s) 
 constexpr int64_t kRowsBwdSmallGrid = 384;  // chunks of 8 rows per lane
 constexpr int64_t kRowsBwdFullLo = 512;     // chunks of 16
 constexpr int64_t kRowsBwdFullHi = 768;
+// 16 rows only where three workgroups' LDS fits a CU: rows of one lane (8 bf16 or
+// 4 fp32 channels) take 80 KB each, two to a CU, and run 8 rows instead.  300
+// training passes of such rows with 513 to 768 chunks of 16: 0.90 of the time with
+// 16 (0.75 to 1.00, one 1.06); bf16 D=8 B=284 H=1 N=4917 112.3 / 89.8 us, D=8 B=46
+// H=6 N=4836 141.2 / 107.1, fp32 D=4 B=37 H=9 N=4754 149.7 / 115.9.
+constexpr size_t kCuLds = 160 << 10;
+
+// Dynamic LDS of scan_rows_bwd (its layout is at the kernel's head).
+size_t rows_bwd_lds(const RowSplit& s, RowShape c, int slots) {
+  const int64_t G = (int64_t)c.NW * (64 / s.lpr), S = slots;
+  return 16 * G * (c.R + 1) + 8 * c.NW + 4 * (G * (S + 1) + 2 * c.NW * S + 3 * S + (G + 1) + (c.R + 1));
+}
 
 // Short sequences as the forward's, with one wavefront only where its 64 lanes
 // hold a stream's channels (slots), and of 8 rows only for many streams
@@ -895,15 +907,15 @@ RowShape rows_bwd_shape(const RowSplit& s, int64_t B, int64_t H, int64_t N, int 
   const int64_t L = rows_chunk(s, RowShape{8, 4}), n = B * H * s.ng;
   if (N <= L) return RowShape{8, 4};
   const int64_t grid16 = (N + 2 * L - 1) / (2 * L) * n;
-  if (grid16 > kRowsBwdFullLo && grid16 <= kRowsBwdFullHi) return RowShape{16, 4};
+  if (grid16 > kRowsBwdFullLo && grid16 <= kRowsBwdFullHi && 3 * rows_bwd_lds(s, RowShape{16, 4}, slots) <= kCuLds)
+    return RowShape{16, 4};
   return RowShape{(N + L - 1) / L * n > kRowsBwdSmallGrid ? 8 : 4, 4};
 }
 
 template <typename T, bool NT>
 int launch_rows_bwd_nt(const RowBwdArgs& ra, int64_t grid, RowShape c, hipStream_t s) {
   const BwdArgs& a = ra.s;
-  const int64_t G = (int64_t)c.NW * ra.gw, S = ra.slots;
-  const size_t lds = 16 * G * (c.R + 1) + 8 * c.NW + 4 * (G * (S + 1) + 2 * c.NW * S + 3 * S + (G + 1) + (c.R + 1));
+  const size_t lds = rows_bwd_lds(RowSplit{ra.lpr, a.ng, true}, c, ra.slots);
   // Windows as launch_bwd's: narrow in several rounds, else by chain length.
   const int64_t resident = 4 * (int64_t)cu_count();
   const bool rounds = resident > 0 && grid > resident;

@@ -245,6 +245,29 @@ def test_rows_backward_grids(hip_device, kdecay_lib, dname, B, H, N, D):
         first = dv, dl
 
 
+def _backward_chunks(lib, dname, B, H, N, D):
+    """Chunks per stream of the row kernels' backward, from the size of its saved states."""
+    n, rest = divmod(lib.kdecay_scan_rows_saved_states_floats(B, H, N, D, CODES[dname]) - 2 * H * N, B * H * D)
+    assert rest == 0
+    return n
+
+
+def test_backward_rows_per_lane_fit_the_lds(kdecay_lib):
+    """Grids of 513 to 768 chunks take 16 rows per lane, for which three
+    workgroups have to fit a CU's LDS: rows of one lane (80 KB a workgroup) take 8."""
+    for dname, D in (("bf16", 8), ("f16", 8), ("f32", 4)):
+        assert _backward_chunks(kdecay_lib, dname, 10, 16, 16384, D) == 8  # 2048 rows: 8 per lane
+    for dname, D in (("bf16", 16), ("f32", 8)):
+        assert _backward_chunks(kdecay_lib, dname, 10, 16, 8192, D) == 4  # 2048 rows: 16 per lane
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname,B,H,N,D", [("bf16", 40, 16, 4000, 8), ("f32", 40, 16, 4000, 4), ("bf16", 10, 16, 8000, 16)])
+def test_rows_backward_of_one_and_two_lanes(hip_device, kdecay_lib, dname, B, H, N, D):
+    """The grids of the test above: 8 rows per lane with one lane per row, 16 with two."""
+    test_rows_backward_grids(hip_device, kdecay_lib, dname, B, H, N, D)
+
+
 @pytest.mark.gpu
 def test_rows_backward_infinite_gradient_stays_in_its_channel(hip_device, kdecay_lib):
     """An infinite gradient at the last row: every earlier row of that channel

@@ -260,6 +260,8 @@ py::object scan(const py::object& lam_o, const py::object& V_o, const py::object
   if (d.index() != c10::hip::current_device()) return py::none();
   const int64_t B = V.size(0), H = V.size(1), N = V.size(2), D = V.size(3);
   const at::ScalarType vt = V.scalar_type();
+  // Not a torch.dtype: the general path, which takes what torch.empty_like does.
+  if (!out_dtype_o.is_none() && !THPDtype_Check(out_dtype_o.ptr())) return py::none();
   const at::ScalarType ot = out_dtype_o.is_none() ? vt : out_dtype_o.cast<at::ScalarType>();
   const int v_code = dtype_code(vt), o_code = dtype_code(ot);
   if (v_code < 0 || (ot != vt && (ot != at::kFloat || vt == at::kDouble))) return py::none();

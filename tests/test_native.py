@@ -93,3 +93,15 @@ def test_step_equals_the_general_path(hip_device, kdecay_lib):
         out, state = torch.empty_like(o, dtype=torch.float32), s.clone()
         r = kilat_amd.decay_step(lam, state, v, pos, out=out, new_state=state)
         assert r[0] is out and r[1] is state and torch.equal(state, n)
+
+
+@pytest.mark.gpu
+def test_out_dtype_that_is_no_torch_dtype(hip_device, kdecay_lib):
+    """What torch.empty_like takes for a dtype is taken (a Python type), and what
+    it refuses is refused with its TypeError."""
+    lam, V = torch.rand(3, device=hip_device), torch.randn(2, 3, 40, 16, dtype=torch.float64, device=hip_device)
+    y = kilat_amd.global_decay_scan(lam, V, out_dtype=float)
+    assert y.dtype == torch.float64 and torch.equal(y, kilat_amd.global_decay_scan(lam, V))
+    for wrong in ("float64", 6, object()):
+        with pytest.raises(TypeError):
+            kilat_amd.global_decay_scan(lam, V, out_dtype=wrong)

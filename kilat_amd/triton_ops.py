@@ -18,28 +18,39 @@ not patched by kilat_amd.integration and keeps Kilat's own function.)
 from __future__ import annotations
 
 import contextlib
+import importlib
 from typing import Optional, Tuple, Union
 
 import torch
 
 from . import _lib
 
-try:
-    from . import _native  # the host path in C++ (csrc/native.cpp)
-except ImportError as e:
-    class _Missing:
-        """Stands in for _native until it is built: any use raises."""
 
-        def __init__(self, why: str) -> None:
-            self.why = why
+def _import_native():
+    importlib.invalidate_caches()  # it may have been built since the last attempt
+    return importlib.import_module(f"{__package__}._native")
 
-        def __getattr__(self, name: str):
+
+class _Unbuilt:
+    """Stands in for _native where it could not be loaded: the first use after it
+    is built (by this process or another) takes its place; any earlier raises."""
+
+    def __getattr__(self, name: str):
+        global _native
+        try:
+            _native = _import_native()
+        except ImportError as e:
             raise RuntimeError(
-                f"kilat_amd: _native.so cannot be loaded ({self.why}); build it with `python -m kilat_amd._build` "
+                f"kilat_amd: _native.so cannot be loaded ({e}); build it with `python -m kilat_amd._build` "
                 "(there is no fallback)"
-            )
+            ) from e
+        return getattr(_native, name)
 
-    _native = _Missing(str(e))
+
+try:
+    _native = _import_native()  # the host path in C++ (csrc/native.cpp)
+except ImportError:
+    _native = _Unbuilt()
 
 _DTYPE_CODE = {
     torch.float32: _lib.KDECAY_F32,

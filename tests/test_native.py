@@ -2,6 +2,11 @@
 read as they are, with the general path's results, and leaves the others to it."""
 from __future__ import annotations
 
+import os
+import shutil
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -31,6 +36,39 @@ def test_cpu_and_foreign_arguments_are_left(kdecay_lib):
     assert _native.decay_step(lam, V[:, :, 0], V[:, :, 0], 3, None, None, torch.float32) is None
     with pytest.raises(RuntimeError, match="cpu"):
         kilat_amd.triton_global_decay(lam, V)
+
+
+def test_package_imported_before_it_is_built(kdecay_lib, tmp_path):
+    """Imported without its libraries the package raises at the first call, and
+    works in the same process once they are there (build() and the fixtures that
+    build import it first)."""
+    src = os.path.dirname(kilat_amd.__file__)
+    pkg = tmp_path / "kilat_amd"
+    pkg.mkdir()
+    for name in os.listdir(src):
+        if name.endswith(".py"):
+            shutil.copy(os.path.join(src, name), pkg)
+    program = """
+import shutil, sys
+import torch, kilat_amd
+assert kilat_amd.__file__.startswith(sys.argv[1]), kilat_amd.__file__
+lam, V = torch.rand(3), torch.randn(2, 3, 5, 64)
+calls = (lambda: kilat_amd.triton_global_decay(lam, V), lambda: kilat_amd.decay_step(lam, V[:, :, 0], V[:, :, 0], 3))
+def error(call):
+    try:
+        call()
+    except RuntimeError as e:
+        return str(e)
+for call in calls:
+    assert "cannot be loaded" in error(call)
+for name in ("libkdecay.so", "_native.so"):
+    shutil.copy(sys.argv[2] + "/" + name, sys.argv[1] + "/kilat_amd/" + name)
+for call in calls:
+    assert "is on cpu" in error(call), error(call)
+"""
+    run = subprocess.run([sys.executable, "-c", program, str(tmp_path), src], capture_output=True, text=True,
+                         env={**os.environ, "PYTHONPATH": str(tmp_path)}, cwd=tmp_path, timeout=300)
+    assert run.returncode == 0, run.stderr
 
 
 @pytest.mark.gpu

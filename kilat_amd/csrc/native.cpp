@@ -160,8 +160,14 @@ struct ScanNode : torch::autograd::Function<ScanNode> {
     // The saved V also feeds the backward kernel, whose addressing takes a
     // narrower range of row strides than the forward's.
     const Tensor Vk = train_layout_ok(V, rows) ? V : V.contiguous();
-    Tensor out = out_dtype == Vk.scalar_type() ? at::empty_like(Vk) : at::empty(Vk.sizes(), Vk.options().dtype(out_dtype));
-    if (!out_layout_ok(out, rows)) out = at::empty(Vk.sizes(), Vk.options().dtype(out_dtype));
+    // y is laid out like V; for head dims of the channel groups contiguous where
+    // its type is another one or the chunked kernels would not take V as it is.
+    const bool group = chunked_head_dim(D, V.element_size());
+    const auto yopt = V.options().dtype(out_dtype);
+    const bool like = !group || (out_dtype == V.scalar_type() && train_layout_ok(V, false));
+    Tensor y = like ? at::empty_like(V, yopt) : at::empty(V.sizes(), yopt);
+    if (group && !out_layout_ok(y, rows)) y = at::empty(V.sizes(), yopt);
+    const Tensor out = out_layout_ok(y, rows) ? y : at::empty(V.sizes(), yopt);  // what the kernel writes
     const Tensor final = at::empty({B, H, D}, Vk.options().dtype(at::kFloat));
     const auto [nstates, nbytes] = train_sizes(B, H, N, D, v_code, rows);
     const Tensor states = at::empty({static_cast<int64_t>(std::max<size_t>(nstates, 1))}, final.options());
@@ -182,11 +188,12 @@ struct ScanNode : torch::autograd::Function<ScanNode> {
                                          t_offset, s),
               "kdecay_scan_fwd_sequential");
     }
+    if (!out.is_same(y)) y.copy_(out);
     ctx->set_materialize_grads(false);
     ctx->saved_data["t_offset"] = t_offset;
     ctx->saved_data["rows"] = rows;
     ctx->save_for_backward({lam, Vk, init32, states});
-    return {out, final};
+    return {y, final};
   }
 
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,

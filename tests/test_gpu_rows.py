@@ -269,6 +269,26 @@ def test_rows_backward_of_one_and_two_lanes(hip_device, kdecay_lib, dname, B, H,
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dname,out,D", [("bf16", "f32", 96), ("bf16", None, 96), ("f16", "f32", 50), ("f64", None, 20),
+                                         ("bf16", "f32", 3)])
+def test_training_output_is_laid_out_like_V(hip_device, kdecay_lib, dname, out, D):
+    """y of a training pass over a head dim off the channel groups has the
+    strides of empty_like(V), also as fp32 of a 2-byte V and where V has a channel
+    stride; the same values as from a contiguous V."""
+    dtype, out = DTYPES[dname], DTYPES[out or dname]
+    lam = lam_uniform(3, 0.5, 0.999, torch.Generator().manual_seed(4)).to(hip_device)
+    wide = torch.randn(2, 130, 3, 2 * D, device=hip_device).to(dtype)
+    for V in (wide[..., :D].contiguous().transpose(1, 2), wide.transpose(1, 2)[..., ::2],
+              wide[..., :D].permute(0, 2, 3, 1).contiguous().transpose(2, 3)):
+        W, C = V.detach().requires_grad_(), V.detach().contiguous().requires_grad_()
+        y, ref = (kilat_amd.global_decay_scan(lam, v, out_dtype=out) for v in (W, C))
+        assert y.dtype == out and torch.equal(y, ref)
+        assert y.stride() == torch.empty_like(V, dtype=out).stride()
+        gy = torch.randn_like(ref)
+        assert torch.equal(torch.autograd.grad(y, W, gy)[0], torch.autograd.grad(ref, C, gy)[0])
+
+
+@pytest.mark.gpu
 def test_rows_backward_infinite_gradient_stays_in_its_channel(hip_device, kdecay_lib):
     """An infinite gradient at the last row: every earlier row of that channel
     is infinite (never NaN from rows past the end), the others are finite, also

@@ -190,23 +190,36 @@ def reserve_workspace(
     dev = torch.device("cuda") if device is None else torch.device(device)
     if dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())
-    code = _dtype_code(torch.empty((), dtype=dtype), "dtype")
-    lib = _lib.load()
-    if chunked_head_dim(D, dtype):
-        nbytes = lib.kdecay_scan_workspace_bytes(B, H, N, D, code)
-    else:
-        nbytes = lib.kdecay_scan_rows_workspace_bytes(B, H, N, D, code)
-    if backward:
-        # float64 is trained through the fp32 kernels (_scan_with_grad)
-        tcode = _lib.KDECAY_F32 if code == _lib.KDECAY_F64 else code
-        tdtype = torch.float32 if code == _lib.KDECAY_F64 else dtype
-        nbytes = max(nbytes, _train_sizes(lib, B, H, N, D, tcode, not chunked_head_dim(D, tdtype))[1])
-    if D <= 32 and _row_vectors_ok(D, dtype):  # narrow heads may take either kernels (narrow_rows in native.cpp)
-        nbytes = max(nbytes, lib.kdecay_scan_rows_workspace_bytes(B, H, N, D, code),
-                     _train_sizes(lib, B, H, N, D, tcode, True)[1] if backward else 0)
+    nbytes = _reserve_bytes(_lib.load(), B, H, N, D, dtype, backward)
     with _on_device(dev):
         ws = _workspace(dev, _stream_ptr(dev), nbytes)
     return 0 if ws is None else ws.numel()
+
+
+def _reserve_bytes(lib, B: int, H: int, N: int, D: int, dtype: torch.dtype, backward: bool) -> int:
+    """Bytes of workspace that scans of this shape, and their backward, can ask for."""
+    code = _dtype_code(torch.empty((), dtype=dtype), "dtype")
+
+    def size(dt: torch.dtype, c: int, train: bool) -> int:
+        rows = _row_vectors_ok(D, dt)
+        # Channel-group kernels, on zero-padded rows where neither kind takes D.
+        Dc = D if chunked_head_dim(D, dt) else 0 if rows else _padded_head_dim(D, dt)
+        n = 0
+        if Dc:
+            n = lib.kdecay_scan_workspace_bytes(B, H, N, Dc, c)
+            if train:
+                n = max(n, _train_sizes(lib, B, H, N, Dc, c, False)[1])
+        # Narrow heads may take either kind (narrow_rows in native.cpp).
+        if rows and (not Dc or D <= 32):
+            n = max(n, lib.kdecay_scan_rows_workspace_bytes(B, H, N, D, c))
+            if train:
+                n = max(n, _train_sizes(lib, B, H, N, D, c, True)[1])
+        return n
+
+    n = size(dtype, code, backward and dtype != torch.float64)
+    if backward and dtype == torch.float64:  # trained through the fp32 kernels (_scan_with_grad)
+        n = max(n, size(torch.float32, _lib.KDECAY_F32, True))
+    return n
 
 
 def workspace_error(V: torch.Tensor, clear: bool = False) -> int:

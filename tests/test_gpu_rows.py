@@ -10,7 +10,7 @@ from kilat_amd import _lib
 from kilat_amd.triton_ops import _row_vectors_ok, chunked_head_dim
 from oracle import decay_oracle as O
 from tests.decay_cases import lam_uniform, rel_err
-from tests.test_gpu_grad import check, gpu_grads, oracle_grads
+from tests.test_gpu_grad import check, gpu_grads, oracle_grads, rel
 
 DTYPES = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16, "f64": torch.float64}
 CODES = {"f32": _lib.KDECAY_F32, "bf16": _lib.KDECAY_BF16, "f16": _lib.KDECAY_F16, "f64": _lib.KDECAY_F64}
@@ -158,6 +158,75 @@ def test_rows_under_capture(hip_device, kdecay_lib):
             kilat_amd.triton_global_decay(lam, V[:, :, :1000, :64])
             side.synchronize()
             assert torch.equal(y, ref)
+
+
+def test_reserved_bytes_cover_the_route_of_every_head_dim(kdecay_lib):
+    """reserve_workspace's size: never less than the row kernels', the
+    channel-group kernels' or, for rows of less than one vector, the padded
+    route's, forward and training."""
+    from kilat_amd.triton_ops import _padded_head_dim, _reserve_bytes
+
+    lib, B, H, N = kdecay_lib, 2, 3, 4096
+    for dname, dtype in DTYPES.items():
+        tname = "f32" if dname == "f64" else dname  # float64 is trained through the fp32 kernels
+        for D in (1, 2, 3, 4, 7, 8, 16, 17, 32, 40, 64, 80, 96, 128, 129, 136):
+            for train, name in ((False, dname), (True, tname)):
+                rows, group = _row_vectors_ok(D, DTYPES[name]), chunked_head_dim(D, DTYPES[name])
+                need = []
+                if rows and not group:
+                    need += [lib.kdecay_scan_rows_workspace_bytes, lib.kdecay_scan_rows_bwd_workspace_bytes][:1 + train]
+                else:
+                    need += [lib.kdecay_scan_workspace_bytes, lib.kdecay_scan_bwd_workspace_bytes][:1 + train]
+                Dk = D if rows or group else _padded_head_dim(D, DTYPES[name])
+                for size in need:
+                    n = size(B, H, N, Dk, CODES[name])
+                    assert 0 < n <= _reserve_bytes(lib, B, H, N, D, dtype, train), (dname, D, train)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname,D", [("bf16", 4), ("f32", 3), ("f16", 80), ("bf16", 16)])
+def test_capture_after_reserve(hip_device, kdecay_lib, dname, D):
+    """On a stream that ran nothing before, reserve_workspace suffices to capture
+    a scan and a training pass; replayed between eager calls of other shapes."""
+    dtype = DTYPES[dname]
+    lam = lam_uniform(3, 0.8, 0.999, torch.Generator().manual_seed(79)).to(hip_device).requires_grad_()
+    V = torch.randn(2, 4000, 3, D, device=hip_device).to(dtype).transpose(1, 2)
+    _captured(lam, V, lambda: kilat_amd.reserve_workspace(2, 3, 4000, D, dtype))
+
+
+def _captured(lam, V, prepare):
+    """A forward and a training pass captured on a new stream after prepare(),
+    every replay against the sequential kernel and an uncaptured backward."""
+    gy = torch.randn_like(V)
+    V = V.detach().requires_grad_()
+    tol = TOL[V.dtype]
+    with torch.no_grad():
+        ref = kilat_amd.global_decay_scan(lam, V, algorithm="sequential")
+    dv0, dl0 = torch.autograd.grad(kilat_amd.triton_global_decay(lam, V), (V, lam), gy)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        prepare()
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            with torch.no_grad():
+                y = kilat_amd.triton_global_decay(lam, V)
+            yt = kilat_amd.triton_global_decay(lam, V)
+            dv, dl = torch.autograd.grad(yt, (V, lam), gy)
+        for _ in range(3):
+            for t in (y, yt, dv, dl):
+                t.detach().zero_()
+            graph.replay()
+            side.synchronize()
+            for t in (y, yt.detach()):
+                assert rel_err(t, ref) <= tol
+            assert rel_err(dv, dv0) <= tol and rel(dl, dl0) <= 1e-4
+            with torch.no_grad():  # eager, on the same workspace
+                small = kilat_amd.triton_global_decay(lam, V[:, :, :100])
+            assert rel_err(small, ref[:, :, :100]) <= tol
+        assert kilat_amd.workspace_error(V) == 0
 
 
 def test_rows_backward_rejects_bad_arguments(kdecay_lib):

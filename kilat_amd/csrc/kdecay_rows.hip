@@ -412,7 +412,11 @@ void scan_rows(RowScanArgs ra) {
 // row's last vector shares with the one before it are computed in both, but
 // count once in dlam: the later vector's copy of V and of the incoming state is
 // zeroed, which zeroes every term of dlam that the lane adds for them, while
-// its dV depends on gy alone.
+// its dV depends on gy alone.  A gy there that is not finite makes dlam NaN
+// (infinity times zero) where the sum alone might be an infinity.  Summing such
+// lanes once more without the copies cost every lane registers the kernels do not
+// have to spare, whole-vector head dims included: 500 training passes at 1.027 of
+// the time (1.135 at most), and at 1.023 (1.112) channel by channel.
 struct RowBwdArgs {
   BwdArgs s;  // ng: streams per head; flags: [nstream][nchunk][slots] words
   int lpr, gw, slots;

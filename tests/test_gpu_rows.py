@@ -402,3 +402,27 @@ def test_narrow_heads_on_the_row_kernels(hip_device, kdecay_lib, dname, D):
     dl0 = sum(p[3].double() for p in parts)
     assert rel_err(y, y0) <= TOL[dtype] and rel_err(fin, fin0) <= 1e-5 and rel_err(dv, dv0) <= TOL[dtype]
     assert float((dl - dl0).abs().max() / dl0.abs().max()) <= 1e-4
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname,D,c", [("bf16", 48, 3), ("bf16", 50, 45), ("f32", 5, 2), ("bf16", 301, 295)])
+def test_rows_backward_infinite_gradient_reaches_dlam(hip_device, kdecay_lib, dname, D, c):
+    """An infinite gradient, of y or of the final state, leaves its head's dlam
+    infinite or NaN (also in a channel that a row's last vector repeats, where
+    it is NaN), the other head's finite and as without it."""
+    lam = torch.tensor([0.5, 0.9], device=hip_device, requires_grad=True)
+    V = torch.randn(1, 2, 402, D, device=hip_device).to(DTYPES[dname]).requires_grad_()
+    gy = torch.randn(1, 2, 402, D, device=hip_device).to(DTYPES[dname])
+    gfin = torch.randn(1, 2, D, device=hip_device)
+
+    def dlam(gy, gfin):
+        y, fin = kilat_amd.global_decay_scan(lam, V, return_final_state=True)
+        return torch.autograd.grad((y, fin), lam, (gy, gfin))[0]
+
+    ref = dlam(gy, gfin)
+    assert torch.isfinite(ref).all()
+    for where in ("y", "final"):
+        g, f = gy.clone(), gfin.clone()
+        (g[:, 0, 200] if where == "y" else f[:, 0])[..., c] = float("inf")
+        dl = dlam(g, f)
+        assert not torch.isfinite(dl[0]) and torch.equal(dl[1], ref[1])

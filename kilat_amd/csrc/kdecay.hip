@@ -1299,26 +1299,46 @@ constexpr int64_t kLongChain = 64;
 // (contiguous D=16 H=4 B=628 N=719: 56.3, 8 x 4 68.5).
 //
 // Sequences of a 128-byte group that leave much of their 512-row chunks empty
-// run in 384-row chunks of 12 rows per lane, as many per stream.  Measured (us,
-// 512-row chunks, in slices where those applied / 384-row; a copy): N=300 B=30
-// 10.5 / 8.7 (5.3), B=80 16.9 / 15.2, B=200 53.0 / 38.1 (35.5); N=360 B=30 10.3 /
-// 9.3, B=80 18.8 / 19.9, B=200 52.6 / 45.1; N=600 B=30 14.7 / 12.4, B=60 29.2 /
-// 25.5, B=128 59.4 / 50.0 (45.5); N=700 B=42 19.5 / 17.3, B=128 60.9 / 54.6; N=768
-// B=60 27.7 / 30.9; N=1100 B=20 16.1 / 13.8, B=64 65.6 / 43.9 (41.7); N=1152 B=28
-// 20.5 / 18.6, B=40 28.0 / 29.0, B=64 56.6 / 44.1; N=1280 (five sixths) B=40 29.3
-// / 31.2.  One chunk per stream in two slices that fill their workgroup slots
-// gains nothing (B=128, two slices of 768: N=270 23.3 / 25.1, N=300 26.7 / 26.4, N=340
-// 26.0 / 29.5), nor do small grids, which keep 8 rows (H=13 B=1 N=331 D=128 6.7 /
-// 7.8; N=700 B=8 7.4 / 8.5; two chunks per stream to 560: H=7 N=655 B=33 10.4 /
-// 11.1), and wide heads (D=256 H=1 B=216 N=611 28.8 / 31.2).  256- and 192-row
-// chunks were up to 13% faster than 384 on grids of several rounds (N=520 B=64
-// 20.7 against 23.9), but need more look-back words than the 512-row chunks did:
-// a workspace sized before could be too small.  Not when the forward saves
-// states: its lanes' ends then have to meet the backward's chunk starts, which
+// run in 384-row chunks of 12 rows per lane, as many per stream.  Measured (bf16
+// D=64 H=12, us, 512-row chunks, in slices where those applied / 384-row; a copy):
+// N=300 B=30 10.5 / 8.7 (5.3), B=200 53.0 / 38.1 (35.5); N=360 B=30 10.3 / 9.3,
+// B=200 52.6 / 45.1; N=600 B=30 14.7 / 12.4, B=60 29.2 / 25.5, B=128 59.4 / 50.0
+// (45.5); N=700 B=42 19.5 / 17.3, B=128 60.9 / 54.6; N=1100 B=20 16.1 / 13.8, B=64
+// 65.6 / 43.9 (41.7); N=1152 B=28 20.5 / 18.6, B=64 56.6 / 44.1; but N=768 B=60
+// 27.7 / 30.9, N=1280 (five sixths) B=40 29.3 / 31.2.  Where they lose (11548
+// shapes of every type, 128- to 512-byte heads and H=1 to 32, each against 512- or
+// 256-row chunks; time with 384 rows as a share of theirs, geometric mean, worst):
+//   - grids of 256-row chunks (chunk_shape: small, or six to a CU with several
+//     groups per head), which fit the length by themselves: two chunks per stream
+//     to 640 1.06, 1.25; several groups, 1025 to 1536 chunks 1.01, 1.14;
+//   - one chunk per stream beyond two to a CU, in one launch (513 to 1024 chunks):
+//     fp32, fp64 and fp32 outputs 0.99, 1.17, 2-byte types below 288 rows 0.96,
+//     1.10 (from there 0.94, 1.04); and in two slices that fill their workgroup
+//     slots (N=340 B=128 26.0 / 29.5) or where the one launch would be a round of
+//     five chunks a CU and part of another: 1281 to 1536 0.97, 1.16;
+//   - three chunks per stream on grids that give some CUs a third chunk, 513 to
+//     576: 0.96, 1.13; in fp64, with its shorter rows, two or three chunks on 513
+//     to 768: 0.99, 1.25;
+//   - fp32 outputs of a contiguous 2-byte V where the 512-row chunks run as slices:
+//     one chunk per stream 1.00, 1.16, two on 1281 to 1536 1.01, 1.07, three to 1536
+//     1.04, 1.16 (from the projection layout 0.92, 0.87 and 0.93);
+//   - sequences that end less than 8 rows into their last 256-row (one chunk per
+//     stream) or 512-row chunk, in one launch: 1.01, 1.20; slices are slower there
+//     (N=516 B=104 61.0 / 36.0).
+// Without those 8924 are left: 0.89, 1.10, half a percent of them above 1.03 (N=1152
+// B=40 H=12: from the projection layout 38.6 / 38.2, contiguous 30.3 / 31.1).
+// 256- and 192-row chunks were up to 13% faster than 384 on grids of several rounds
+// (N=520 B=64 20.7 against 23.9), but need more look-back words than the 512-row
+// chunks did: a workspace sized before could be too small.  Not when the forward
+// saves states: its lanes' ends then have to meet the backward's chunk starts, which
 // are no multiples of 12 rows.
 constexpr int kRTiny = 4;
 constexpr int kRFit = 12;
-constexpr int64_t kFitGrid2 = 560;
+constexpr int64_t kFitPast = 8;
+constexpr int64_t kFitHalf = 288;
+constexpr int64_t kFitTwo = 512;     // two chunks on every CU
+constexpr int64_t kFitRound = 1280;  // five
+constexpr int64_t kFitUneven = 576, kFitUneven64 = 768;
 
 constexpr int64_t kSliceRound = 1024;
 constexpr int64_t kSliceCUs = 256;
@@ -1347,19 +1367,38 @@ int64_t slice_count(int64_t B, int64_t per_b, bool* fill) {
   return best;
 }
 
-// N rows in `chain` chunks of 512 (gw row groups per wavefront: 8), `grid` of
-// them in all, `slices`: run as batch slices otherwise.
-bool fit_rows(int64_t B, int64_t N, int64_t gw, int64_t chain, int64_t grid, bool slices) {
-  const int64_t l12 = kNW * gw * kRFit, p16 = chain * kNW * gw * kR;
-  if ((N + l12 - 1) / l12 != chain) return false;
-  if (chain >= 3) return 4 * N <= 3 * p16 && grid > kSmallGrid;
-  if (chain == 2) return 100 * N <= 72 * p16 && grid > kFitGrid2;
-  if (grid <= kSmallGrid1 || 100 * N > 71 * p16) return false;
-  if (slices) {
+// fp32 outputs of a 2-byte V (wide), and whether V's rows are adjacent in memory.
+struct FwdOut {
+  bool wide = false, adjacent = false;
+};
+
+// A grid of 512-row chunks (chunk_shape) and its arrays.
+struct FitGrid {
+  int64_t chain, grid;      // chunks per stream and in all
+  bool slices;              // runs as batch slices otherwise
+  int es;                   // bytes of an element
+  FwdOut out;
+};
+
+// Whether N rows run in 384-row chunks (gw row groups per wavefront: 8).
+bool fit_rows(int64_t B, int64_t N, int64_t gw, const FitGrid& f) {
+  const int64_t l12 = kNW * gw * kRFit, l16 = kNW * gw * kR, p16 = f.chain * l16;
+  if ((N + l12 - 1) / l12 != f.chain) return false;
+  if (!f.slices && N - (f.chain - 1) * l16 < (f.chain == 1 ? l16 / 2 : 0) + kFitPast) return false;
+  const bool part = f.grid > kFitRound && f.grid <= kSixHi;
+  if (f.slices && f.chain == 1 && part) return false;
+  if (f.slices && f.out.wide && f.out.adjacent && (f.chain == 1 || part || (f.chain >= 3 && f.grid <= kSixHi)))
+    return false;
+  if (f.chain >= 2 && f.grid > kFitTwo && f.grid <= (f.es == 8 ? kFitUneven64 : kFitUneven)) return false;
+  if (f.chain >= 3) return 4 * N <= 3 * p16;
+  if (f.chain == 2) return 100 * N <= 72 * p16;
+  if (100 * N > 71 * p16) return false;
+  if (f.slices) {
     bool fill;
-    return slice_count(B, grid / B, &fill) > 2 || !fill;
+    return slice_count(B, f.grid / B, &fill) > 2 || !fill;
   }
-  return grid <= 720 || 10 * N <= 6 * p16 || grid > 1024;
+  if (f.grid <= kFitTwo || f.grid > kSixHi) return true;
+  return f.grid <= kSliceRound && f.es == 2 && !f.out.wide && N >= kFitHalf;
 }
 
 // Row groups per wavefront of the forward's streams.
@@ -1367,7 +1406,7 @@ int64_t row_groups(int v_dtype, int64_t D) { return 64 / (group_width(v_dtype, D
 
 // saves: the launch saves the backward's states (more than one backward chunk
 // per stream).
-ChunkShape chunk_shape(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves) {
+ChunkShape chunk_shape(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves, FwdOut out) {
   const int64_t gw = row_groups(v_dtype, D);
   const bool full = group_width(v_dtype, D) * elem_size(v_dtype) == 128;
   if (N <= gw * kRTiny) return ChunkShape{kRTiny, 1};
@@ -1381,14 +1420,16 @@ ChunkShape chunk_shape(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, 
   const int64_t grid = chain * nstream;
   const int64_t lim = chain == 1 ? kSmallGrid1 : chain == 2 ? kSmallGrid2 : kSmallGrid;
   const bool wide = full && ng >= kSixWideGroups && chain <= kSixWideChain && grid >= kSixWideLo;
-  if (full && !saves && !wide && fit_rows(B, N, gw, chain, grid, sliceable(B, chain, H * chain, ng)))
+  const bool six = full && chain <= kSixChain && grid > (ng > 1 ? kSixLoGroups : kSixLo) && grid <= kSixHi;
+  const bool slices = sliceable(B, chain, H * chain, ng);
+  if (full && !saves && !wide && grid > lim && (!six || slices) &&
+      fit_rows(B, N, gw, FitGrid{chain, grid, slices, elem_size(v_dtype), out}))
     return ChunkShape{kRFit, kNW};
   if (grid <= lim) {
     const int64_t chain8 = (N + L / 2 - 1) / (L / 2);  // chunks per stream at 8 rows per lane
     return full && chain8 >= kLongChain ? ChunkShape{kRSmall, kNWLong} : ChunkShape{kRSmall, kNWSmall};
   }
-  if (full && chain <= kSixChain && grid > (ng > 1 ? kSixLoGroups : kSixLo) && grid <= kSixHi)
-    return ChunkShape{kRSmall, kNWSmall, true};
+  if (six) return ChunkShape{kRSmall, kNWSmall, true};
   if (wide) return ChunkShape{kRSmall, kNWSmall, true};
   return ChunkShape{kR, kNW};
 }
@@ -1426,7 +1467,7 @@ ChunkShape chunk_shape(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, 
 // slots (B=72 H=12: one launch 163.8, 8 slices of 864 chunks 167.6; B=80 in 8
 // of 960: 181.7 / 172.6; B=56 in 7 of 768: 129.2 / 122.8).
 // Only sequences that chunk_shape leaves in 512-row chunks.
-int64_t fwd_slices(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves) {
+int64_t fwd_slices(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves, FwdOut out) {
   const int64_t DG = group_width(v_dtype, D);
   if (B < 2 || DG != D || DG * elem_size(v_dtype) != 128) return 1;
   const int64_t gw = row_groups(v_dtype, D);
@@ -1435,7 +1476,7 @@ int64_t fwd_slices(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool
   const int64_t chain = (N + L - 1) / L;
   const int64_t per_b = H * chain;  // 512-row chunks of one batch element
   if (!sliceable(B, chain, per_b, 1)) return 1;
-  if (!saves && fit_rows(B, N, gw, chain, B * per_b, true)) return 1;
+  if (!saves && fit_rows(B, N, gw, FitGrid{chain, B * per_b, true, elem_size(v_dtype), out})) return 1;
   bool fill;
   const int64_t n = slice_count(B, per_b, &fill);
   return B * per_b >= 4 * kSliceRound && !fill ? 1 : n;
@@ -1885,7 +1926,8 @@ uint32_t kdecay_debug_fastdiv(uint32_t n, uint32_t d, int want_mod) {
   return want_mod ? f.mod(n) : f.div(n);
 }
 
-// How the forward runs a shape, with or without saved states.
+// How the forward runs a shape, with or without saved states.  Wide outputs take
+// the plan of the one or of the other (fit_rows refuses more of them).
 struct FwdPlan {
   int64_t nslice;    // launches, over balanced slices of the batch
   ChunkShape shape;
@@ -1893,10 +1935,10 @@ struct FwdPlan {
   size_t need;       // workspace bytes: slices run one after another on it, so the largest one's
 };
 
-static FwdPlan fwd_plan(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves) {
+static FwdPlan fwd_plan(int64_t B, int64_t H, int64_t N, int64_t D, int v_dtype, bool saves, FwdOut out = {}) {
   FwdPlan p;
-  p.nslice = fwd_slices(B, H, N, D, v_dtype, saves);
-  p.shape = p.nslice > 1 ? ChunkShape{kR, kNW} : chunk_shape(B, H, N, D, v_dtype, saves);
+  p.nslice = fwd_slices(B, H, N, D, v_dtype, saves, out);
+  p.shape = p.nslice > 1 ? ChunkShape{kR, kNW} : chunk_shape(B, H, N, D, v_dtype, saves, out);
   p.L = chunk_rows(v_dtype, D, p.shape);
   p.nchunk = (N + p.L - 1) / p.L;
   const int64_t Bs = (B + p.nslice - 1) / p.nslice;
@@ -1950,7 +1992,7 @@ static int scan_fwd_impl(const void* V, int v_dtype, const int64_t* v_strides, v
   float2* const rowtab = saved ? reinterpret_cast<float2*>(saved + B * H * D * nsaved) : nullptr;
   // A workspace of less than kdecay_scan_workspace_bytes, but enough for a
   // saving launch's shapes, takes those.
-  FwdPlan plan = fwd_plan(B, H, N, D, v_dtype, saved != nullptr);
+  FwdPlan plan = fwd_plan(B, H, N, D, v_dtype, saved != nullptr, FwdOut{out_dtype != v_dtype, v_strides[2] == D});
   if (workspace_bytes < plan.need && !saved) plan = fwd_plan(B, H, N, D, v_dtype, true);
   const int64_t L = plan.L, nchunk = plan.nchunk, nslice = plan.nslice;
   const bool multi = nchunk > 1;

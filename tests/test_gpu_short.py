@@ -49,6 +49,38 @@ def test_short_sequences(hip_device, kdecay_lib, dname, out, D, unit):
     assert rel_err(y, ref) <= TOL[y.dtype]
 
 
+def test_384_row_chunks_where_batch_slices_would_run(kdecay_lib):
+    """384-row chunks in one launch take more words than the slices of 512-row
+    chunks they replace: up to 72% of two chunks and three quarters of three."""
+    lib = kdecay_lib
+    for B, N, fit in ((100, 700, True), (64, 1025, True), (64, 1152, True), (64, 1153, False), (64, 513, True),
+                      (64, 737, True), (64, 738, False)):
+        sizes = [f(B, 12, N, 64, _lib.KDECAY_BF16)
+                 for f in (lib.kdecay_scan_workspace_bytes, lib.kdecay_scan_workspace_least_bytes)]
+        assert (sizes[0] > sizes[1]) == fit, (B, N)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname,out,H,D,N,streams", [
+    ("bf16", None, 1, 64, 300, (160, 161, 512, 513)),             # one chunk per stream: small, two to a CU, more
+    ("f32", None, 1, 64, 264, (255, 256, 257, 769)),              # two groups per head; the shortest length
+    ("bf16", "f32", 1, 64, 350, (500, 1030, 1600)),               # fp32 outputs, also in slices
+    ("f16", None, 2, 64, 700, (320, 322, 516)),                   # two chunks: 640, 644, 1032
+    ("bf16", None, 1, 128, 600, (162, 256, 258, 384, 386)),       # two groups: 648, 1024, 1032, 1536, 1544
+    ("f64", None, 1, 16, 1100, (139, 171, 256, 257)),             # fp64: 417, 513, 768, 771
+    ("f16", "f32", 1, 64, 1100, (170, 171, 214, 342, 512, 513)),  # three chunks: 510, 513, 642, slices from 1026
+])
+def test_384_row_chunk_edges(hip_device, kdecay_lib, dname, out, H, D, N, streams):
+    """Either side of the lines of 384-row chunks, against the sequential kernel."""
+    for n in streams:
+        lam = lam_uniform(H, 0.5, 0.9999, torch.Generator().manual_seed(n)).to(hip_device)
+        V = torch.randn(n // H, H, N, D, device=hip_device).to(DTYPES[dname])
+        kw = dict(return_final_state=True, out_dtype=DTYPES[out] if out else None)
+        y, fin = kilat_amd.global_decay_scan(lam, V, **kw)
+        ys, fs = kilat_amd.global_decay_scan(lam, V, algorithm="sequential", **kw)
+        assert rel_err(y, ys) <= TOL[y.dtype] and rel_err(fin, fs) <= 1e-5, n
+
+
 @pytest.mark.gpu
 def test_small_workspace_takes_the_saving_shapes(hip_device, kdecay_lib):
     """A workspace of kdecay_scan_workspace_least_bytes, less than

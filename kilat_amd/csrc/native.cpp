@@ -83,10 +83,33 @@ bool bwd_rows_fit(int64_t N, int64_t D, int64_t es, int64_t row_stride) {
 // 13.1; 32.9 / 24.5, contiguous 13.2 / 13.6 and B=32 H=16 N=1000 contiguous 17.5 /
 // 18.9; 26.2 / 29.4; fp32 D=16 B=8 H=12 N=4096 view 16.9 / 14.0; 32.2 / 26.0; but
 // B=2 H=6 N=1024 bf16 D=32 view 7.9 / 7.8; 10.3 / 11.6.
-bool narrow_rows(const Tensor& V) {
-  const int64_t D = V.size(3), es = V.element_size();
-  if (D > 32 || D * es >= 128 || V.numel() * es < (4 << 20)) return false;
-  return V.stride(2) != D || D * es == 32;
+//
+// Where they lose among those (7483 forwards and training passes; time as a share
+// of the chunked kernels', geometric mean, worst), for few (b,h) streams, whose
+// chains are long and whose grids leave CUs idle, mostly:
+//   - 64-byte rows, forward, fewer than 40 streams: to 8192 rows 1.01, 1.15; past
+//     32256 rows where the grid is small (chunks of 8 wavefronts, rows_shape) 0.97, 1.13;
+//   - 64-byte rows, training: fewer than 40 streams past 16384 rows, in fp32 up to
+//     2^20 rows in all 0.96, 1.11, in 16 bits past 32768 rows with fewer than 24
+//     streams 0.98, 1.07; 513 to 640 rows (a second backward chunk of 512, nearly
+//     empty) 0.99, 1.10;
+//   - 32-byte rows: fewer than 24 streams in less than 8 MiB 0.99, 1.13; fp32
+//     outputs of a contiguous 2-byte V past 1024 rows, forward 1.00, 1.11.
+// Without those 6729 are left: 0.72, 1.13, half a percent of them above 1.03.
+//
+// train: a pass with a backward (whose forward goes with it).  wide: fp32 outputs of a
+// 2-byte V.
+bool narrow_rows(const Tensor& V, bool train, bool wide) {
+  const int64_t N = V.size(2), D = V.size(3), es = V.element_size(), streams = V.size(0) * V.size(1);
+  const int64_t bytes = V.numel() * es;
+  if (D > 32 || D * es >= 128 || bytes < (4 << 20)) return false;
+  const bool view = V.stride(2) != D;
+  if (D * es == 32) return (streams >= 24 || bytes >= (8 << 20)) && (view || train || !wide || N <= 1024);
+  if (!view) return false;
+  if (!train) return streams >= 40 || (N > 8192 && (N <= 32256 || streams * N > 416 * 1024));
+  if (N > 512 && N <= 640) return false;
+  if (streams >= 40 || N <= 16384) return true;
+  return es == 2 ? streams >= 24 || N <= 32768 : streams * N > (1 << 20);
 }
 
 bool train_layout_ok(const Tensor& t, bool rows) {
@@ -277,11 +300,12 @@ py::object scan(const py::object& lam_o, const py::object& V_o, const py::object
   const int64_t t_offset = PyLong_AsLongLongAndOverflow(t_offset_o.ptr(), &overflow);
   if (overflow) return py::none();
 
-  const bool narrow = narrow_rows(V), chunked = chunked_head_dim(D, V.element_size()) && !narrow;
+  const bool train = at::GradMode::is_enabled() &&
+                     (V.requires_grad() || lam.requires_grad() || (init.defined() && init.requires_grad()));
+  const bool chunked = chunked_head_dim(D, V.element_size()) && !narrow_rows(V, train, ot != vt);
   if (!chunked && !row_vectors_ok(D, V.element_size())) return py::none();
   const hipStream_t s = stream_of(d);
-  if (at::GradMode::is_enabled() &&
-      (V.requires_grad() || lam.requires_grad() || (init.defined() && init.requires_grad()))) {
+  if (train) {
     if (vt == at::kDouble) return py::none();
     // The workspace is checked before the node is made: where it has to grow,
     // the caller decides what a stream capture does.
@@ -393,5 +417,5 @@ PYBIND11_MODULE(_native, m) {
   m.def("row_vectors_ok", &row_vectors_ok);
   m.def("vector_layout_ok", &vector_layout_ok);
   m.def("bwd_rows_fit", &bwd_rows_fit);
-  m.def("narrow_rows", &narrow_rows);
+  m.def("narrow_rows", &narrow_rows, py::arg("V"), py::arg("train") = false, py::arg("wide") = false);
 }

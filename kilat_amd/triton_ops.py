@@ -355,7 +355,7 @@ def _scan(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, a
             )
             _lib.check(rc, "kdecay_scan_fwd_sequential")
         elif (chunked_head_dim(D, V.dtype) and _vector_layout_ok(V) and _vector_layout_ok(out)
-              and not _native.narrow_rows(V)):
+              and not _native.narrow_rows(V, wide=o_code != v_code)):
             _chunked(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev)
         elif _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev):
             pass
@@ -434,7 +434,7 @@ def _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, d
 def _rows_train(V: torch.Tensor) -> bool:
     """Whether a training pass over V takes the row kernels (see _rows)."""
     B, H, N, D = V.shape
-    if chunked_head_dim(D, V.dtype) and not _native.narrow_rows(V):
+    if chunked_head_dim(D, V.dtype) and not _native.narrow_rows(V, train=True):
         return False
     if not _row_vectors_ok(D, V.dtype):
         return False

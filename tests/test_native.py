@@ -38,6 +38,32 @@ def test_cpu_and_foreign_arguments_are_left(kdecay_lib):
         kilat_amd.triton_global_decay(lam, V)
 
 
+def test_narrow_heads_that_take_the_row_kernels(kdecay_lib):
+    """Either side of the lines of narrow_rows, in the projection layout unless
+    said; smaller than 4 MiB and rows of a whole memory line never."""
+    from kilat_amd import _native
+
+    def takes(B, H, N, D, dname="bf16", contiguous=False, **kw):
+        V = torch.empty((B, H, N, D) if contiguous else (B, N, H, D), dtype=DTYPES[dname])
+        return _native.narrow_rows(V if contiguous else V.transpose(1, 2), **kw)
+
+    assert takes(8, 12, 1500, 32) and not takes(8, 12, 600, 32) and not takes(8, 12, 1500, 32, contiguous=True)
+    assert not takes(8, 12, 1500, 64) and not takes(8, 12, 1500, 32, "f32") and takes(8, 12, 1500, 16, "f32")
+    for N, fwd, train in ((3000, False, True), (8192, False, True), (8193, True, True), (32256, True, True)):
+        assert takes(3, 13, N, 32) == fwd and takes(3, 13, N, 32, train=True) == train, N
+    assert takes(5, 8, 2000, 32) and not takes(1, 12, 33000, 32) and takes(1, 13, 33000, 32)  # by streams, by rows in all
+    assert takes(2, 10, 32768, 32, train=True) and not takes(2, 10, 32769, 32, train=True)
+    assert takes(2, 12, 32769, 32, train=True)
+    assert takes(2, 10, 16384, 16, "f32", train=True) and not takes(2, 10, 16385, 16, "f32", train=True)
+    assert takes(2, 19, 28000, 16, "f32", train=True) and takes(4, 10, 16385, 16, "f32", train=True)
+    for N, train in ((512, True), (513, False), (640, False), (641, True)):
+        assert takes(20, 8, N, 32) and takes(20, 8, N, 32, train=True) == train, N
+    assert takes(2, 12, 6000, 16) and not takes(1, 23, 6000, 16) and takes(1, 23, 12000, 16)
+    assert takes(8, 12, 2000, 16, contiguous=True) and takes(8, 12, 2000, 16, wide=True)
+    assert takes(16, 12, 1024, 16, contiguous=True, wide=True) and not takes(16, 12, 1025, 16, contiguous=True, wide=True)
+    assert takes(8, 12, 2000, 16, contiguous=True, wide=True, train=True)
+
+
 def test_package_imported_before_it_is_built(kdecay_lib, tmp_path):
     """Imported without its libraries the package raises at the first call, and
     works in the same process once they are there (build() and the fixtures that

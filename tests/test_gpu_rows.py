@@ -140,8 +140,7 @@ def test_rows_misaligned_views_and_out(hip_device, kdecay_lib):
 @pytest.mark.gpu
 def test_rows_under_capture(hip_device, kdecay_lib):
     """Captured after reserve_workspace and replayed between eager calls of
-    other shapes on the same workspace; on a stream whose workspace is too
-    small for the row kernel the capture still takes what it took before it."""
+    other shapes on the same workspace, the same bits."""
     g = torch.Generator().manual_seed(78)
     lam = lam_uniform(3, 0.8, 0.999, g).to(hip_device)
     V = torch.randn(2, 3, 3000, 80, generator=g).to(torch.bfloat16).to(hip_device)
@@ -227,6 +226,44 @@ def _captured(lam, V, prepare):
                 small = kilat_amd.triton_global_decay(lam, V[:, :, :100])
             assert rel_err(small, ref[:, :, :100]) <= tol
         assert kilat_amd.workspace_error(V) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,D,kind", [(20, 10, 230, 80, "padded"), (40, 12, 2000, 16, "narrow"),
+                                          (20, 10, 2000, 16, "narrow"), (100, 12, 700, 64, "misaligned")])
+def test_capture_on_a_workspace_too_small_for_the_row_kernels(hip_device, kdecay_lib, B, H, N, D, kind):
+    """Where the stream's workspace holds what the route before the row kernels
+    needs (zero-padding, the channel-group kernels on a view or on a copy) but
+    not what they need, a capture takes that route, forward and training."""
+    from kilat_amd.triton_ops import _padded_head_dim, _stream_ptr, _train_sizes, _workspace
+
+    lib, code = kdecay_lib, _lib.KDECAY_BF16
+    Dk = D if kind != "padded" else _padded_head_dim(D, torch.bfloat16)
+    least = lib.kdecay_scan_workspace_least_bytes(B, H, N, Dk, code)
+    rows = lib.kdecay_scan_rows_workspace_bytes(B, H, N, D, code)
+    train, rows_train = (_train_sizes(lib, B, H, N, d, code, r)[1] for d, r in ((Dk, False), (D, True)))
+    assert least < rows or train < rows_train
+    lam = lam_uniform(H, 0.8, 0.999, torch.Generator().manual_seed(80)).to(hip_device).requires_grad_()
+    V = torch.randn(B, N, H, D + (kind == "misaligned"), device=hip_device).to(torch.bfloat16).transpose(1, 2)
+    V = V[..., 1:] if kind == "misaligned" else V
+    if kind == "misaligned":  # trained through a copy in any case: the forward alone
+        with torch.no_grad():
+            ref = kilat_amd.global_decay_scan(lam, V, algorithm="sequential")
+            side = torch.cuda.Stream()
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side):
+                _workspace(hip_device, _stream_ptr(hip_device), least)
+                side.synchronize()
+                graph = torch.cuda.CUDAGraph()
+                with torch.cuda.graph(graph, stream=side):
+                    y = kilat_amd.triton_global_decay(lam, V)
+                for _ in range(3):
+                    y.zero_()
+                    graph.replay()
+                    side.synchronize()
+                    assert rel_err(y, ref) <= TOL[torch.bfloat16]
+        return
+    _captured(lam, V, lambda: _workspace(hip_device, _stream_ptr(hip_device), max(least, train)))
 
 
 def test_rows_backward_rejects_bad_arguments(kdecay_lib):
@@ -426,3 +463,133 @@ def test_rows_backward_infinite_gradient_reaches_dlam(hip_device, kdecay_lib, dn
         (g[:, 0, 200] if where == "y" else f[:, 0])[..., c] = float("inf")
         dl = dlam(g, f)
         assert not torch.isfinite(dl[0]) and torch.equal(dl[1], ref[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,D", [(1, 16, 32768, 80), (2, 8, 30000, 50), (40, 10, 3000, 96)])
+def test_rows_give_up_is_flagged_not_hung(hip_device, kdecay_lib, B, H, N, D):
+    """The row kernels' look-backs give up after one poll (the library's test
+    hook): every launch returns and sets the error word, the one that gave up
+    writes NaN where it has no carry, and every later one NaN everywhere until the
+    workspace is cleared; then the first launch's bits.  16 streams, and 400, which
+    count toward the epoch's advance through sub-counts."""
+    lam = lam_uniform(H, 0.99, 0.9999, torch.Generator().manual_seed(44)).to(hip_device)
+    V = torch.randn(B, N, H, D, device=hip_device).to(torch.bfloat16).transpose(1, 2)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+
+    def call():
+        y, fin = kilat_amd.global_decay_scan(lam, V, return_final_state=True)
+        torch.cuda.synchronize()
+        return y, fin, kilat_amd.workspace_error(V)
+
+    with torch.cuda.stream(stream):
+        ref, fref, err = call()
+        assert err == 0 and bool(torch.isfinite(ref).all())
+        kdecay_lib.kdecay_debug_set_spin_limit(1)
+        gave_up = False
+        try:
+            for k in range(3):
+                print(f"  forced give-up launch {k}", flush=True)
+                y, fin, err = call()
+                if gave_up:
+                    assert bool(torch.isnan(y).all()) and bool(torch.isnan(fin).all()), k
+                elif err:
+                    assert bool(torch.isnan(y).any()), k
+                    gave_up = True
+                else:
+                    assert torch.equal(y, ref), k
+        finally:
+            kdecay_lib.kdecay_debug_set_spin_limit(0)
+        assert gave_up
+        y, fin, err = call()
+        assert bool(torch.isnan(y).all()) and bool(torch.isnan(fin).all()) and err == 1
+        assert kilat_amd.workspace_error(V, clear=True) == 1
+        for _ in range(2):  # the epoch advances again
+            y, fin, err = call()
+            assert err == 0 and torch.equal(y, ref) and torch.equal(fin, fref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,D", [(2, 4, 16384, 96), (16, 16, 1024, 80), (40, 10, 500, 50)])
+def test_rows_backward_give_up_is_flagged_not_hung(hip_device, kdecay_lib, B, H, N, D):
+    """The training pass likewise: its forward's and its reverse look-back and the
+    wait for a head's dlam partials.  8 streams (the first chunk of each counts
+    toward the epoch's advance), 256 and 400 (the head-summing workgroups and the
+    last of each XCD do)."""
+    g = torch.Generator().manual_seed(45)
+    lam = lam_uniform(H, 0.9, 0.9999, g)
+    V = torch.randn(B, H, N, D, generator=g).to(torch.bfloat16)
+    gy = torch.randn(B, H, N, D, generator=g).to(torch.bfloat16)
+    probe = V[:, :, :1].to(hip_device)  # selects the workspace of this device and stream
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+
+    def call():
+        dv, dl, _ = gpu_grads(lam, V, gy, hip_device)
+        return dv, dl, kilat_amd.workspace_error(probe)
+
+    with torch.cuda.stream(stream):
+        dv0, dl0, err = call()
+        assert err == 0
+        kdecay_lib.kdecay_debug_set_spin_limit(1)
+        gave_up = False
+        try:
+            for k in range(3):
+                print(f"  forced give-up backward {k}", flush=True)
+                dv, dl, err = call()
+                if gave_up:
+                    assert bool(torch.isnan(dv).all()) and bool(torch.isnan(dl).all()), k
+                elif err:
+                    assert bool(torch.isnan(dv).any()) or bool(torch.isnan(dl).any()), k
+                    gave_up = True
+        finally:
+            kdecay_lib.kdecay_debug_set_spin_limit(0)
+        assert gave_up
+        dv, dl, err = call()
+        assert bool(torch.isnan(dv).all()) and bool(torch.isnan(dl).all()) and err == 1
+        assert kilat_amd.workspace_error(probe, clear=True) == 1
+        for _ in range(2):
+            dv, dl, err = call()
+            assert err == 0 and torch.equal(dv, dv0) and torch.equal(dl, dl0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,N,D", [(2, 4, 3000, 80), (25, 10, 700, 96), (40, 10, 900, 50), (2, 3, 90, 80)])
+def test_rows_training_pass_replays_from_a_graph(hip_device, kdecay_lib, B, H, N, D):
+    """A training pass on the row kernels, captured and replayed with eager passes
+    and scans on the same workspace between the replays: the eager bits every
+    time (look-back words and dlam partials are tagged with the launch epoch).
+    8, 250 and 400 streams of several chunks, and one chunk per stream."""
+    g = torch.Generator().manual_seed(46)
+    lam = lam_uniform(H, 0.5, 0.999, g).to(hip_device).requires_grad_()
+    V = torch.randn(B, H, N, D, generator=g).to(torch.bfloat16).to(hip_device).requires_grad_()
+    gy = torch.randn(B, H, N, D, generator=g).to(torch.bfloat16).to(hip_device)
+    init = torch.randn(B, H, D, generator=g).to(hip_device).requires_grad_()
+
+    def launch():
+        y, fin = kilat_amd.global_decay_scan(lam, V, initial_state=init, return_final_state=True, t_offset=5)
+        return (y, *torch.autograd.grad((y, fin), (V, lam, init), (gy, fin.detach())))
+
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        ref = [t.detach().clone() for t in launch()]  # eager first: creates the workspace outside the capture
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = launch()
+        torch.cuda.synchronize()
+        for r in range(4):
+            print(f"  training graph replay {r} N={N} D={D}", flush=True)
+            for t in out:
+                t.detach().zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(a.detach(), b) for a, b in zip(out, ref)), r
+            again = launch()
+            with torch.no_grad():
+                kilat_amd.triton_global_decay(lam, V[:, :, : N // 2])
+            torch.cuda.synchronize()
+            assert all(torch.equal(a.detach(), b) for a, b in zip(again, ref)), r
+        assert kilat_amd.workspace_error(V) == 0

@@ -227,9 +227,9 @@ struct ScanNode : torch::autograd::Function<ScanNode> {
     const int64_t t_offset = ctx->saved_data["t_offset"].toInt();
     const int64_t B = V.size(0), H = V.size(1), N = V.size(2), D = V.size(3);
     const int code = dtype_code(V.scalar_type());
-    Tensor gy = grads[0].defined() ? grads[0].to(V.scalar_type()) : at::zeros_like(V);
+    Tensor gy = grads[0].defined() ? grads[0].to(V.scalar_type()).resolve_neg() : at::zeros_like(V);
     if (!train_layout_ok(gy, rows)) gy = gy.contiguous();
-    const Tensor gfin = grads[1].defined() ? grads[1].to(at::kFloat).contiguous() : Tensor();
+    const Tensor gfin = grads[1].defined() ? grads[1].to(at::kFloat).resolve_neg().contiguous() : Tensor();
     Tensor dV = at::empty_like(V);
     if (!out_layout_ok(dV, rows)) dV = at::empty(V.sizes(), V.options());
     const auto fopt = V.options().dtype(at::kFloat);
@@ -270,9 +270,10 @@ bool plain_state(const Tensor& s, int64_t B, int64_t H, int64_t D, const at::Dev
          s.is_contiguous() && s.device() == d;
 }
 
-// A torch.Tensor or Parameter itself: subclasses go through Python, where their
-// __torch_function__ applies.
-bool plain_tensor(PyObject* o) { return THPVariable_CheckExact(o); }
+// A torch.Tensor or Parameter itself, whose memory holds its values: subclasses go
+// through Python, where their __torch_function__ applies, and so do views that are
+// negated when read (the imaginary part of a conjugate).
+bool plain_tensor(PyObject* o) { return THPVariable_CheckExact(o) && !THPVariable_Unpack(o).is_neg(); }
 
 // global_decay_scan(lam, V, ...) into a new y, for arguments the kernels read as
 // they are; None (nothing launched) otherwise.

@@ -248,8 +248,8 @@ def _lam32(lam: torch.Tensor, H: int, device: torch.device) -> torch.Tensor:
     if lam.numel() != H:
         raise ValueError(f"kilat_amd: lam_scores has {lam.numel()} elements, V has {H} heads")
     if lam.dtype == torch.float32 and lam.dim() == 1 and lam.is_contiguous() and lam.device == device:
-        return lam  # only its memory is read
-    return lam.detach().reshape(H).to(device=device, dtype=torch.float32).contiguous()
+        return lam.resolve_neg()  # only its memory is read
+    return lam.detach().resolve_neg().reshape(H).to(device=device, dtype=torch.float32).contiguous()
 
 
 def _train_sizes(lib, B: int, H: int, N: int, D: int, v_code: int, rows: bool) -> Tuple[int, int]:
@@ -321,6 +321,11 @@ def _scan(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, a
     v_code = _dtype_code(V, "V")
     B, H, N, D = V.shape
     dev = V.device
+    lam, V, initial_state = (t.resolve_neg() if isinstance(t, torch.Tensor) else t for t in (lam, V, initial_state))
+    if isinstance(out, torch.Tensor) and out.is_neg():
+        y, final = _scan(lam, V, initial_state, True, t_offset, torch.empty_like(out), out_dtype, algorithm)
+        out.copy_(y)
+        return (out, final) if return_final_state else out
     if _needs_grad(lam, V, initial_state):
         return _scan_with_grad(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, algorithm)
     lam32 = _lam32(lam, H, dev)
@@ -555,11 +560,11 @@ def decay_step(
     if v_t.numel() != B * H * D:
         raise ValueError(f"kilat_amd: v_t has {v_t.numel()} elements, expected B*H*D={B * H * D}")
     v_code = _dtype_code(v_t, "v_t")
-    vk = v_t.detach().reshape(B, H, D).contiguous()
+    vk = v_t.detach().resolve_neg().reshape(B, H, D).contiguous()
     if v_code == _lib.KDECAY_F64:  # the step kernel takes v_t as fp32 (rounded once), as every type
         vk, v_code = vk.float(), _lib.KDECAY_F32
     lam32 = _lam32(lam, H, dev)
-    s_in = past_state.detach()
+    s_in = past_state.detach().resolve_neg()
     if s_in.dtype != torch.float32 or not s_in.is_contiguous():
         s_in = s_in.to(torch.float32).contiguous()
     if new_state is None:

@@ -169,3 +169,38 @@ def test_out_dtype_that_is_no_torch_dtype(hip_device, kdecay_lib):
     for wrong in ("float64", 6, object()):
         with pytest.raises(TypeError):
             kilat_amd.global_decay_scan(lam, V, out_dtype=wrong)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 80, 16, 3])
+def test_lazily_negated_views(hip_device, kdecay_lib, D):
+    """Tensors whose memory holds their negation (torch._neg_view, the imaginary
+    part of a conjugate) give what their values give: every input, out= and the
+    upstream gradients."""
+    lam = lam_uniform(3, 0.5, 0.9999, torch.Generator().manual_seed(D)).to(hip_device).requires_grad_()
+    V, gy = (torch.randn(2, 3, 70, D, device=hip_device) for _ in range(2))
+    init, gfin = (torch.randn(2, 3, D, device=hip_device) for _ in range(2))
+
+    def neg(t):
+        t = torch._neg_view(-t)
+        assert t.is_neg()
+        return t
+
+    def call(view, algorithm="chunked"):
+        v, i = view(V).requires_grad_(), view(init).requires_grad_()
+        r = kilat_amd.global_decay_scan(lam, v, initial_state=i, return_final_state=True, algorithm=algorithm)
+        return (*r, *torch.autograd.grad(r, (v, lam, i), (view(gy), view(gfin))))
+
+    for algorithm in ("chunked", "sequential"):
+        for a, b in zip(call(neg, algorithm), call(torch.clone, algorithm)):
+            assert torch.equal(a, b)
+        with torch.no_grad():
+            ref = kilat_amd.global_decay_scan(lam, V, initial_state=init, algorithm=algorithm)
+            out = neg(torch.zeros_like(V))
+            y = kilat_amd.global_decay_scan(neg(lam), neg(V), initial_state=neg(init), out=out, algorithm=algorithm)
+            assert y is out and torch.equal(out, ref)
+    with torch.no_grad():
+        assert torch.equal(kilat_amd.triton_global_decay(lam, neg(V)), kilat_amd.triton_global_decay(lam, V))
+    for a, b in zip(kilat_amd.decay_step(neg(lam.detach()), neg(init), neg(gfin), 5),
+                    kilat_amd.decay_step(lam.detach(), init, gfin, 5)):
+        assert torch.equal(a, b)

@@ -307,7 +307,7 @@ py::object scan(const py::object& lam_o, const py::object& V_o, const py::object
   if (!chunked && !row_vectors_ok(D, V.element_size())) return py::none();
   const hipStream_t s = stream_of(d);
   if (train) {
-    if (vt == at::kDouble) return py::none();
+    if (vt == at::kDouble || V.is_inference()) return py::none();
     // The workspace is checked before the node is made: where it has to grow,
     // the caller decides what a stream capture does.
     const size_t nbytes = train_sizes(B, H, N, D, v_code, !chunked).second;

@@ -505,6 +505,9 @@ def _scan_with_grad(lam, V, initial_state, return_final_state, t_offset, out, ou
     o_dtype = out_dtype or V.dtype
     if o_dtype not in (V.dtype, torch.float32):
         raise TypeError("kilat_amd: out dtype must be V's dtype or float32")
+    group = chunked_head_dim(D, V.dtype)
+    if V.is_inference() and not group:
+        V = V.clone()  # an inference tensor cannot be saved for the backward
     y, final = _native.scan_train(lam32, V, init32, int(t_offset), o_dtype, _rows_train(V), algorithm == "sequential")
     if return_final_state:
         return y, final

@@ -204,3 +204,21 @@ def test_lazily_negated_views(hip_device, kdecay_lib, D):
     for a, b in zip(kilat_amd.decay_step(neg(lam.detach()), neg(init), neg(gfin), 5),
                     kilat_amd.decay_step(lam.detach(), init, gfin, 5)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_training_pass_over_an_inference_tensor(hip_device, kdecay_lib):
+    """V made under inference_mode: head dims off the channel groups take it (through
+    a copy, which the backward can keep), those of the groups refuse it."""
+    lam = torch.tensor([0.5, 0.9], device=hip_device, requires_grad=True)
+    for D in (80, 64):
+        V = torch.randn(2, 2, 50, D, device=hip_device)
+        with torch.inference_mode():
+            W = V.clone()
+        if D == 64:
+            with pytest.raises(RuntimeError, match="[Ii]nference"):
+                kilat_amd.triton_global_decay(lam, W)
+            continue
+        y, z = kilat_amd.triton_global_decay(lam, V), kilat_amd.triton_global_decay(lam, W)
+        assert torch.equal(y, z)
+        assert torch.equal(torch.autograd.grad(z.sum(), lam)[0], torch.autograd.grad(y.sum(), lam)[0])

@@ -509,6 +509,9 @@ def _scan_with_grad(lam, V, initial_state, return_final_state, t_offset, out, ou
     if V.is_inference() and not group:
         V = V.clone()  # an inference tensor cannot be saved for the backward
     y, final = _native.scan_train(lam32, V, init32, int(t_offset), o_dtype, _rows_train(V), algorithm == "sequential")
+    kind = type(V.detach())
+    if kind is not torch.Tensor and (o_dtype == V.dtype or not group):
+        y = y.as_subclass(kind)  # as empty_like(V) is
     if return_final_state:
         return y, final
     return y

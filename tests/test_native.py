@@ -207,6 +207,25 @@ def test_lazily_negated_views(hip_device, kdecay_lib, D):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 80, 3])
+def test_training_pass_keeps_a_tensor_subclass(hip_device, kdecay_lib, D):
+    """The result is of V's class, as without a gradient, and of a Parameter a
+    plain tensor; the values and gradients are the plain tensor's."""
+    class Sub(torch.Tensor):
+        pass
+
+    lam = torch.tensor([0.5, 0.9], device=hip_device, requires_grad=True)
+    V, gy = torch.randn(2, 2, 50, D, device=hip_device, requires_grad=True), torch.randn(2, 2, 50, D, device=hip_device)
+    y = kilat_amd.triton_global_decay(lam, V)
+    z = kilat_amd.triton_global_decay(lam, V.as_subclass(Sub))
+    assert type(z) is Sub and torch.equal(z.as_subclass(torch.Tensor), y)
+    assert type(kilat_amd.triton_global_decay(lam.detach(), V.detach().as_subclass(Sub))) is Sub
+    assert type(kilat_amd.triton_global_decay(lam, torch.nn.Parameter(V.detach()))) is torch.Tensor
+    for a, b in zip(torch.autograd.grad(z, (V, lam), gy), torch.autograd.grad(y, (V, lam), gy)):
+        assert torch.equal(a.as_subclass(torch.Tensor), b)
+
+
+@pytest.mark.gpu
 def test_training_pass_over_an_inference_tensor(hip_device, kdecay_lib):
     """V made under inference_mode: head dims off the channel groups take it (through
     a copy, which the backward can keep), those of the groups refuse it."""

@@ -271,6 +271,29 @@ def _workspace_short_in_capture(dev: torch.device, stream: int, nbytes: int) -> 
     return (nbytes if ws is None else nbytes - ws.numel()) > 0 and torch.cuda.is_current_stream_capturing()
 
 
+def _extent(t: torch.Tensor) -> Tuple[int, int]:
+    """First and one past the last byte of t's elements."""
+    last = sum((n - 1) * st for n, st in zip(t.shape, t.stride())) if t.numel() else -1
+    return t.data_ptr(), t.data_ptr() + (last + 1) * t.element_size()
+
+
+def _meets(out: torch.Tensor, V: torch.Tensor, *others) -> bool:
+    """Whether memory of `out` may be read by other workgroups after one has
+    written it: `out` shares a byte range with V, other than being the very same
+    view (each workgroup reads its rows before it writes them), or with another
+    input."""
+    lo, hi = _extent(out)
+
+    def shares(t) -> bool:
+        if not isinstance(t, torch.Tensor) or not t.is_cuda:
+            return False
+        a, b = _extent(t)
+        return a < hi and lo < b
+
+    same = out.data_ptr() == V.data_ptr() and out.stride() == V.stride() and out.dtype == V.dtype
+    return (not same and shares(V)) or any(shares(t) for t in others)
+
+
 def _needs_grad(*ts) -> bool:
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in ts)
 
@@ -322,7 +345,7 @@ def _scan(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, a
     B, H, N, D = V.shape
     dev = V.device
     lam, V, initial_state = (t.resolve_neg() if isinstance(t, torch.Tensor) else t for t in (lam, V, initial_state))
-    if isinstance(out, torch.Tensor) and out.is_neg():
+    if isinstance(out, torch.Tensor) and (out.is_neg() or _meets(out, V, lam, initial_state)):
         y, final = _scan(lam, V, initial_state, True, t_offset, torch.empty_like(out), out_dtype, algorithm)
         out.copy_(y)
         return (out, final) if return_final_state else out
@@ -420,7 +443,9 @@ def _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, d
     if _workspace_short_in_capture(dev, stream, nbytes):
         return False
     Vk = V if V.stride(3) == 1 else V.contiguous()
-    outk = out if out.stride(3) == 1 else torch.empty(V.shape, dtype=out.dtype, device=dev)
+    # An out whose elements share memory goes through out.copy_, which refuses it.
+    once = out.stride(3) == 1 and not any(st == 0 and n > 1 for st, n in zip(out.stride(), out.shape))
+    outk = out if once else torch.empty(V.shape, dtype=out.dtype, device=dev)
     ws = _workspace(dev, stream, nbytes)
     rc = lib.kdecay_scan_fwd_rows(
         Vk.data_ptr(), v_code, _lib.strides4(Vk.stride()),

@@ -137,6 +137,51 @@ def test_rows_misaligned_views_and_out(hip_device, kdecay_lib):
         assert rel_err(W, ref) <= TOL[torch.bfloat16]
 
 
+def test_outputs_that_meet_an_input():
+    """Which out= the kernels may not write directly: any that shares a byte range
+    with an input, but V itself."""
+    from kilat_amd.triton_ops import _meets
+
+    class Dev(torch.Tensor):  # the check looks at addresses alone
+        is_cuda = True
+
+    def meets(out, V, *others):
+        return _meets(*(t.as_subclass(Dev) if t is not None else None for t in (out, V, *others)))
+
+    buf = torch.empty(2, 3, 11, 40)
+    V = buf[:, :, 1:]
+    assert not meets(V, V) and not meets(buf[:, :, 1:], V)
+    assert meets(buf[:, :, :-1], V)  # shifted by a row
+    assert meets(V.transpose(2, 3), V) and meets(V.view(torch.int32), V)
+    assert not meets(torch.empty(2, 3, 10, 40), V)
+    assert not meets(buf[1:], buf[:1]) and not meets(buf[:1], buf[1:])  # side by side
+    lam, init = buf[0, 1, 5, :3], buf[:, :, 0]
+    assert not meets(torch.empty(2, 3, 10, 40), V, lam, init) and meets(V, V, lam) and meets(V, V, None, init)
+    assert not meets(buf[:, :, :0], V)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,base", [(80, 0), (50, 0), (64, 1), (64, 0)])
+def test_out_that_overlaps_an_input(hip_device, kdecay_lib, D, base):
+    """out= shifted by a row against V, over the carried state, and over one head
+    only (several rows in the same memory, refused off the channel groups)."""
+    lam = lam_uniform(4, 0.8, 0.999, torch.Generator().manual_seed(81)).to(hip_device)
+    big = torch.randn(2, 4, 901, D + base, device=hip_device).to(torch.bfloat16)
+    keep = big.clone()
+    V, room = big[:, :, 1:, base:], big[:, :, :-1, base:]
+    ref = kilat_amd.triton_global_decay(lam, V.clone())
+    assert kilat_amd.global_decay_scan(lam, V, out=room) is room and rel_err(room, ref) <= TOL[torch.bfloat16]
+    big.copy_(keep)
+    f = torch.randn(2, 4, 30, D, device=hip_device)
+    init, W = f[:, :, 0], torch.randn(2, 4, 30, D, device=hip_device)
+    ref = kilat_amd.global_decay_scan(lam, W, initial_state=init.clone())
+    kilat_amd.global_decay_scan(lam, W, initial_state=init, out=f)
+    assert rel_err(f, ref) <= TOL[torch.float32]
+    if D != 64:
+        with pytest.raises(RuntimeError):
+            kilat_amd.global_decay_scan(lam, W, out=torch.empty(2, 1, 30, D, device=hip_device).expand(2, 4, 30, D))
+
+
 @pytest.mark.gpu
 def test_rows_under_capture(hip_device, kdecay_lib):
     """Captured after reserve_workspace and replayed between eager calls of

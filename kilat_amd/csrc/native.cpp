@@ -233,7 +233,7 @@ struct ScanNode : torch::autograd::Function<ScanNode> {
     Tensor dV = at::empty_like(V);
     if (!out_layout_ok(dV, rows)) dV = at::empty(V.sizes(), V.options());
     const auto fopt = V.options().dtype(at::kFloat);
-    const Tensor dlam = at::empty({H}, fopt);
+    const Tensor dlam = V.numel() ? at::empty({H}, fopt) : at::zeros({H}, fopt);  // nothing to sum: no launch writes it
     const Tensor dinit = init.defined() ? at::empty({B, H, D}, fopt) : Tensor();
     {
       const c10::DeviceGuard guard(V.device());

@@ -241,3 +241,17 @@ def test_training_pass_over_an_inference_tensor(hip_device, kdecay_lib):
         y, z = kilat_amd.triton_global_decay(lam, V), kilat_amd.triton_global_decay(lam, W)
         assert torch.equal(y, z)
         assert torch.equal(torch.autograd.grad(z.sum(), lam)[0], torch.autograd.grad(y.sum(), lam)[0])
+
+
+@pytest.mark.gpu
+def test_gradients_of_an_empty_batch(hip_device, kdecay_lib):
+    """No sequences, or no rows: dlam is zero."""
+    for D in (64, 80, 3):
+        for B, N in ((0, 5), (2, 0)):
+            lam = torch.tensor([0.5, 0.9, 0.7], device=hip_device, requires_grad=True)
+            V = torch.empty(B, 3, N, D, device=hip_device, requires_grad=True)
+            y = kilat_amd.triton_global_decay(lam, V)
+            junk = torch.full((3,), float("nan"), device=hip_device)
+            del junk  # what an uninitialised dlam would be made of
+            dl, dv = torch.autograd.grad(y, (lam, V), torch.empty_like(y))
+            assert torch.equal(dl, torch.zeros_like(dl)) and dv.shape == V.shape

@@ -255,3 +255,151 @@ def test_gradients_of_an_empty_batch(hip_device, kdecay_lib):
             del junk  # what an uninitialised dlam would be made of
             dl, dv = torch.autograd.grad(y, (lam, V), torch.empty_like(y))
             assert torch.equal(dl, torch.zeros_like(dl)) and dv.shape == V.shape
+
+
+def _train_inputs(dev, D, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    lam = lam_uniform(2, 0.5, 0.999, g).to(dev).requires_grad_()
+    V, gy = (torch.randn(2, 2, 300, D, generator=g).to(dev) for _ in range(2))
+    return lam, V.requires_grad_(), gy
+
+
+def _grads(y, lam, V, gy):
+    return torch.autograd.grad(y, (V, lam), gy)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 80])
+def test_node_under_saved_tensor_hooks_and_checkpointing(hip_device, kdecay_lib, D):
+    """Saved tensors that are packed elsewhere (copies, the host) or dropped and
+    computed again give the same bits."""
+    from torch.utils.checkpoint import checkpoint
+
+    f = kilat_amd.triton_global_decay
+    lam, V, gy = _train_inputs(hip_device, D)
+    ref = _grads(f(lam, V), lam, V, gy)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t.clone(), lambda t: t):
+        y = f(lam, V)
+    assert any(t.data_ptr() == V.data_ptr() for t in packed)
+    results = [_grads(y, lam, V, gy)]
+    with torch.autograd.graph.save_on_cpu():
+        y = f(lam, V)
+    results += [_grads(y, lam, V, gy), _grads(checkpoint(f, lam, V, use_reentrant=False), lam, V, gy)]
+    W = V.detach().clone().requires_grad_()
+    checkpoint(f, lam, W, use_reentrant=True).backward(gy)
+    results.append((W.grad, lam.grad))
+    for dv, dl in results:
+        assert torch.equal(dv, ref[0]) and torch.equal(dl, ref[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 80])
+def test_node_refusals(hip_device, kdecay_lib, D):
+    """What the node cannot do raises: a second backward, V changed in place
+    before the backward, functorch transforms, forward mode.  A backward with
+    create_graph gives gradients without a graph."""
+    import torch.autograd.forward_ad as fwad
+
+    f = kilat_amd.triton_global_decay
+    lam, V, gy = _train_inputs(hip_device, D)
+    y = f(lam, V)
+    _grads(y, lam, V, gy)
+    with pytest.raises(RuntimeError, match="second time"):
+        _grads(y, lam, V, gy)
+    W = V * 1
+    y = f(lam, W)
+    W.add_(1)
+    with pytest.raises(RuntimeError, match="inplace"):
+        _grads(y, lam, V, gy)
+    W, plain = V.detach(), lam.detach()
+    for call in (lambda: torch.func.grad(lambda v: f(plain, v).sum())(W), lambda: torch.func.vjp(lambda v: f(plain, v), W),
+                 lambda: torch.func.jvp(lambda v: f(plain, v), (W,), (gy,)),
+                 lambda: torch.func.vmap(lambda v: f(plain, v))(torch.stack([W, W])),
+                 lambda: torch.func.vmap(lambda v: kilat_amd.decay_step(plain, W[:, :, 0], v, 3)[0])(gy[:, :, :2].movedim(2, 0))):
+        with pytest.raises(RuntimeError):
+            call()
+    with fwad.dual_level(), pytest.raises(RuntimeError):
+        f(lam, fwad.make_dual(V, gy))
+    dv, dl = torch.autograd.grad(f(lam, V), (V, lam), gy.clone().requires_grad_(), create_graph=True)
+    assert not dv.requires_grad and not dl.requires_grad
+
+
+@pytest.mark.gpu
+def test_compiled_callers_break_the_graph_and_agree(hip_device, kdecay_lib):
+    lam, V, gy = _train_inputs(hip_device, 64)
+    step = (lam.detach(), V.detach()[:, :, 0].contiguous(), V.detach()[:, :, 1].contiguous(), 3)
+    torch._dynamo.reset()
+    for backend in ("eager", "aot_eager"):
+        f = torch.compile(lambda a, v: 2 * kilat_amd.triton_global_decay(a, v * 1), backend=backend)
+        y, ref = f(lam, V), 2 * kilat_amd.triton_global_decay(lam, V * 1)
+        assert torch.equal(y, ref)
+        for a, b in zip(_grads(y, lam, V, gy), _grads(ref, lam, V, gy)):
+            assert torch.equal(a, b)
+        g = torch.compile(lambda *a: kilat_amd.decay_step(*a)[0] + 1, backend=backend)
+        assert torch.equal(g(*step), kilat_amd.decay_step(*step)[0] + 1)
+    torch._dynamo.reset()
+
+
+@pytest.mark.gpu
+def test_threads_on_their_own_streams(hip_device, kdecay_lib):
+    """Scans, training passes and steps from several threads at once, each on its
+    own stream (and so its own workspace), give what one thread gives."""
+    import threading
+
+    data = [_train_inputs(hip_device, D, seed) for seed, D in enumerate((64, 80, 64, 50))]
+
+    def work(lam, V, gy):
+        y = kilat_amd.triton_global_decay(lam, V)
+        with torch.no_grad():
+            z, fin = kilat_amd.global_decay_scan(lam, V, return_final_state=True)
+        s = kilat_amd.decay_step(lam.detach(), fin, gy[:, :, 0].contiguous(), 300)
+        return (y.detach(), *_grads(y, lam, V, gy), z, fin, *s)
+
+    ref = [work(*d) for d in data]
+    torch.cuda.synchronize()
+    errors = []
+
+    def run(k):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(20):
+                    out = work(*data[k])
+                    torch.cuda.current_stream().synchronize()
+                    assert all(torch.equal(a, b) for a, b in zip(out, ref[k]))
+        except BaseException as e:  # noqa: B036 - reported by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(len(data))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    assert not errors and not any(t.is_alive() for t in threads), errors
+
+
+@pytest.mark.gpu
+def test_first_calls_of_two_threads(hip_device, kdecay_lib):
+    """The first calls of a process, made by several threads at the same time,
+    return (the workspace table is looked up once, which may let another thread run)."""
+    program = """
+import threading, torch, kilat_amd
+lam, V = torch.rand(3, device="cuda"), torch.randn(2, 3, 3000, 64, device="cuda")
+W, barrier, out = V.clone().requires_grad_(), threading.Barrier(6), []
+def run(k):
+    with torch.cuda.stream(torch.cuda.Stream()):
+        barrier.wait()
+        y = kilat_amd.triton_global_decay(lam, W if k % 2 else V)
+        torch.cuda.current_stream().synchronize()
+        out.append(y.detach())
+torch.cuda.synchronize()
+threads = [threading.Thread(target=run, args=(k,), daemon=True) for k in range(6)]
+for t in threads: t.start()
+for t in threads: t.join(60)
+assert len(out) == 6
+ref = kilat_amd.global_decay_scan(lam, V, algorithm="sequential")
+assert all(((y - ref).abs().max() / ref.abs().max()).item() < 1e-5 for y in out)
+"""
+    root = os.path.dirname(os.path.dirname(kilat_amd.__file__))
+    run = subprocess.run([sys.executable, "-c", program], cwd=root, capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0, run.stderr

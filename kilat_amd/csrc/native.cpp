@@ -118,6 +118,20 @@ bool train_layout_ok(const Tensor& t, bool rows) {
 
 bool out_layout_ok(const Tensor& t, bool rows) { return rows ? t.stride(3) == 1 : vector_layout_ok(t); }
 
+// Whether a scan from V into out goes to the channel-group kernels as they are.
+bool chunked_route(const Tensor& V, const Tensor& out) {
+  return chunked_head_dim(V.size(3), V.element_size()) && vector_layout_ok(V) && vector_layout_ok(out) &&
+         !narrow_rows(V, false, out.scalar_type() != V.scalar_type());
+}
+
+// Whether the row kernels write `out` directly: adjacent channels, and no two
+// elements in the same memory (Tensor::copy_ refuses those).
+bool rows_out_ok(const Tensor& out) {
+  for (int64_t k = 0; k < 3; ++k)
+    if (out.stride(k) == 0 && out.size(k) > 1) return false;
+  return out.stride(3) == 1;
+}
+
 void check(int rc, const char* what) {
   TORCH_CHECK(rc == 0, "kilat_amd: ", what, " failed (code ", rc, "): ", kdecay_last_error_string());
 }
@@ -275,6 +289,41 @@ bool plain_state(const Tensor& s, int64_t B, int64_t H, int64_t D, const at::Dev
 // negated when read (the imaginary part of a conjugate).
 bool plain_tensor(PyObject* o) { return THPVariable_CheckExact(o) && !THPVariable_Unpack(o).is_neg(); }
 
+// First byte and one past the last of a tensor's elements.
+std::pair<uintptr_t, uintptr_t> extent(const Tensor& t) {
+  const uintptr_t p = reinterpret_cast<uintptr_t>(t.const_data_ptr());
+  if (t.numel() == 0) return {p, p};
+  int64_t last = 0;
+  for (int64_t k = 0; k < t.dim(); ++k) last += (t.size(k) - 1) * t.stride(k);
+  return {p, p + (last + 1) * t.element_size()};
+}
+
+// Whether memory of `out` may be read by other workgroups after one has written
+// it: `out` shares a byte range with V, other than being the very same view (each
+// workgroup reads its rows before it writes them), or with another input.
+bool meets(const Tensor& out, const Tensor& V, const Tensor& lam, const std::optional<Tensor>& init) {
+  const auto [lo, hi] = extent(out);
+  const auto shares = [lo = lo, hi = hi](const Tensor& t) {
+    const auto [a, b] = extent(t);
+    return a < hi && lo < b;
+  };
+  const bool same = out.const_data_ptr() == V.const_data_ptr() && out.strides() == V.strides() &&
+                    out.scalar_type() == V.scalar_type();
+  return (!same && shares(V)) || shares(lam) || (init.has_value() && shares(*init));
+}
+
+// Whether the kernels can read these tensors and write `out` as they lie: none
+// lazily negated, and out apart from the inputs.  Anything but a tensor is left to
+// the checks that follow.
+bool as_they_lie(const py::object& lam_o, const py::object& V_o, const py::object& init_o, const py::object& out_o) {
+  for (PyObject* o : {lam_o.ptr(), V_o.ptr(), init_o.ptr(), out_o.ptr()})
+    if (THPVariable_Check(o) && THPVariable_Unpack(o).is_neg()) return false;
+  if (!THPVariable_Check(out_o.ptr()) || !THPVariable_Check(V_o.ptr()) || !THPVariable_Check(lam_o.ptr())) return true;
+  const bool has_init = THPVariable_Check(init_o.ptr());
+  return !meets(THPVariable_Unpack(out_o.ptr()), THPVariable_Unpack(V_o.ptr()), THPVariable_Unpack(lam_o.ptr()),
+                has_init ? std::optional<Tensor>(THPVariable_Unpack(init_o.ptr())) : std::nullopt);
+}
+
 // global_decay_scan(lam, V, ...) into a new y, for arguments the kernels read as
 // they are; None (nothing launched) otherwise.
 py::object scan(const py::object& lam_o, const py::object& V_o, const py::object& init_o, bool want_final,
@@ -414,6 +463,10 @@ PYBIND11_MODULE(_native, m) {
   m.def("scan", &scan);
   m.def("decay_step", &decay_step);
   m.def("scan_train", &scan_train, py::call_guard<py::gil_scoped_release>());
+  m.def("chunked_route", &chunked_route);
+  m.def("rows_out_ok", &rows_out_ok);
+  m.def("as_they_lie", &as_they_lie);
+  m.def("meets", &meets);
   m.def("chunked_head_dim", &chunked_head_dim);
   m.def("row_vectors_ok", &row_vectors_ok);
   m.def("vector_layout_ok", &vector_layout_ok);

@@ -248,8 +248,8 @@ def _lam32(lam: torch.Tensor, H: int, device: torch.device) -> torch.Tensor:
     if lam.numel() != H:
         raise ValueError(f"kilat_amd: lam_scores has {lam.numel()} elements, V has {H} heads")
     if lam.dtype == torch.float32 and lam.dim() == 1 and lam.is_contiguous() and lam.device == device:
-        return lam.resolve_neg()  # only its memory is read
-    return lam.detach().resolve_neg().reshape(H).to(device=device, dtype=torch.float32).contiguous()
+        return lam  # only its memory is read
+    return lam.detach().reshape(H).to(device=device, dtype=torch.float32).contiguous()
 
 
 def _train_sizes(lib, B: int, H: int, N: int, D: int, v_code: int, rows: bool) -> Tuple[int, int]:
@@ -269,29 +269,6 @@ def _workspace_short_in_capture(dev: torch.device, stream: int, nbytes: int) -> 
     nbytes (it cannot grow there)."""
     ws = _workspaces.get((dev.index, stream))
     return (nbytes if ws is None else nbytes - ws.numel()) > 0 and torch.cuda.is_current_stream_capturing()
-
-
-def _extent(t: torch.Tensor) -> Tuple[int, int]:
-    """First and one past the last byte of t's elements."""
-    last = sum((n - 1) * st for n, st in zip(t.shape, t.stride())) if t.numel() else -1
-    return t.data_ptr(), t.data_ptr() + (last + 1) * t.element_size()
-
-
-def _meets(out: torch.Tensor, V: torch.Tensor, *others) -> bool:
-    """Whether memory of `out` may be read by other workgroups after one has
-    written it: `out` shares a byte range with V, other than being the very same
-    view (each workgroup reads its rows before it writes them), or with another
-    input."""
-    lo, hi = _extent(out)
-
-    def shares(t) -> bool:
-        if not isinstance(t, torch.Tensor) or not t.is_cuda:
-            return False
-        a, b = _extent(t)
-        return a < hi and lo < b
-
-    same = out.data_ptr() == V.data_ptr() and out.stride() == V.stride() and out.dtype == V.dtype
-    return (not same and shares(V)) or any(shares(t) for t in others)
 
 
 def _needs_grad(*ts) -> bool:
@@ -344,11 +321,12 @@ def _scan(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, a
     v_code = _dtype_code(V, "V")
     B, H, N, D = V.shape
     dev = V.device
-    lam, V, initial_state = (t.resolve_neg() if isinstance(t, torch.Tensor) else t for t in (lam, V, initial_state))
-    if isinstance(out, torch.Tensor) and (out.is_neg() or _meets(out, V, lam, initial_state)):
-        y, final = _scan(lam, V, initial_state, True, t_offset, torch.empty_like(out), out_dtype, algorithm)
-        out.copy_(y)
-        return (out, final) if return_final_state else out
+    if not _native.as_they_lie(lam, V, initial_state, out):
+        lam, V, initial_state = (t.resolve_neg() if isinstance(t, torch.Tensor) else t for t in (lam, V, initial_state))
+        if out is not None:
+            y, final = _scan(lam, V, initial_state, True, t_offset, torch.empty_like(out), out_dtype, algorithm)
+            out.copy_(y)
+            return (out, final) if return_final_state else out
     if _needs_grad(lam, V, initial_state):
         return _scan_with_grad(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, algorithm)
     lam32 = _lam32(lam, H, dev)
@@ -382,8 +360,7 @@ def _scan(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, a
                 final.data_ptr() if final is not None else None, B, H, N, D, int(t_offset), stream,
             )
             _lib.check(rc, "kdecay_scan_fwd_sequential")
-        elif (chunked_head_dim(D, V.dtype) and _vector_layout_ok(V) and _vector_layout_ok(out)
-              and not _native.narrow_rows(V, wide=o_code != v_code)):
+        elif _native.chunked_route(V, out):
             _chunked(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev)
         elif _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, dev):
             pass
@@ -443,9 +420,7 @@ def _rows(lib, V, v_code, out, o_code, lam32, init32, final, t_offset, stream, d
     if _workspace_short_in_capture(dev, stream, nbytes):
         return False
     Vk = V if V.stride(3) == 1 else V.contiguous()
-    # An out whose elements share memory goes through out.copy_, which refuses it.
-    once = out.stride(3) == 1 and not any(st == 0 and n > 1 for st, n in zip(out.stride(), out.shape))
-    outk = out if once else torch.empty(V.shape, dtype=out.dtype, device=dev)
+    outk = out if _native.rows_out_ok(out) else torch.empty(V.shape, dtype=out.dtype, device=dev)
     ws = _workspace(dev, stream, nbytes)
     rc = lib.kdecay_scan_fwd_rows(
         Vk.data_ptr(), v_code, _lib.strides4(Vk.stride()),
@@ -590,12 +565,14 @@ def decay_step(
     _require_hip(v_t, "v_t")
     if v_t.numel() != B * H * D:
         raise ValueError(f"kilat_amd: v_t has {v_t.numel()} elements, expected B*H*D={B * H * D}")
+    if not _native.as_they_lie(lam, past_state, v_t, None):
+        lam, past_state, v_t = (t.resolve_neg() if isinstance(t, torch.Tensor) else t for t in (lam, past_state, v_t))
     v_code = _dtype_code(v_t, "v_t")
-    vk = v_t.detach().resolve_neg().reshape(B, H, D).contiguous()
+    vk = v_t.detach().reshape(B, H, D).contiguous()
     if v_code == _lib.KDECAY_F64:  # the step kernel takes v_t as fp32 (rounded once), as every type
         vk, v_code = vk.float(), _lib.KDECAY_F32
     lam32 = _lam32(lam, H, dev)
-    s_in = past_state.detach().resolve_neg()
+    s_in = past_state.detach()
     if s_in.dtype != torch.float32 or not s_in.is_contiguous():
         s_in = s_in.to(torch.float32).contiguous()
     if new_state is None:

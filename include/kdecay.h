@@ -106,6 +106,9 @@ enum {
  *                affected.)  It may be NULL when
  *                kdecay_scan_workspace_bytes() returns 0.
  *
+ * out may be V itself (its address, strides and type); otherwise the memory of
+ * out and final_state must be apart from every input's.
+ *
  * Requirements of this (vector) path: D = 16, 32, or a multiple of 64 (bf16,
  * fp16), 32 (fp32) or 16 (fp64) channels; d-stride 1; 16-byte aligned V and
  * out; the other strides multiples of 16 bytes.
@@ -135,8 +138,9 @@ size_t kdecay_scan_workspace_least_bytes(int64_t B, int64_t H, int64_t N,
  * is any number of channels of at least one 16-byte vector (8 bf16/fp16, 4
  * fp32, 2 fp64), and V, out and the other strides need the element type's
  * alignment only (d-stride 1).  Streams are whole rows of up to 256 bytes; it
- * is for the arrays kdecay_scan_fwd refuses, which is the faster one for
- * those it takes.
+ * is for the arrays kdecay_scan_fwd refuses, which is the faster one for those
+ * it takes but for some heads of 16 and 32 channels whose rows are part of a
+ * 128-byte line (narrow_rows in kilat_amd/csrc/native.cpp says which).
  */
 int kdecay_scan_fwd_rows(const void* V, int v_dtype, const int64_t* v_strides,
                          void* out, int out_dtype, const int64_t* out_strides,

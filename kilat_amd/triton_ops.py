@@ -299,10 +299,12 @@ def global_decay_scan(
     on the row kernel, rows of less than 16 bytes zero-padded to the next head
     dim the chunked kernels take.  When lam, V or initial_state
     requires grad, the result carries a backward for every head dim, layout,
-    algorithm and out= (the gradients always come from the chunked backward
-    kernel).  The backward kernel takes the upstream gradient in V's dtype:
-    with out_dtype=float32 for a bf16/fp16 V, that gradient is rounded to V's
-    dtype first.  A float64 V takes float64 out only; with a gradient it runs
+    algorithm and out= (the gradients come from the chunked backward kernels,
+    of the channel groups or of rows, also with algorithm="sequential").  It
+    keeps V, not a copy: changing V in place before the backward raises, as for
+    any saved tensor.  The backward kernels take the upstream gradient in V's
+    dtype: with out_dtype=float32 for a bf16/fp16 V, that gradient is rounded to
+    V's dtype first.  A float64 V takes float64 out only; with a gradient it runs
     the fp32 training kernels on V rounded to fp32.
     """
     if out is None and algorithm == "chunked":

@@ -323,6 +323,7 @@ def _scan(lam, V, initial_state, return_final_state, t_offset, out, out_dtype, a
     v_code = _dtype_code(V, "V")
     B, H, N, D = V.shape
     dev = V.device
+    # Negated views, and an out in which other workgroups still read an input: through copies.
     if not _native.as_they_lie(lam, V, initial_state, out):
         lam, V, initial_state = (t.resolve_neg() if isinstance(t, torch.Tensor) else t for t in (lam, V, initial_state))
         if out is not None:
